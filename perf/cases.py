@@ -1,0 +1,496 @@
+"""The work this library is used for, as cases that can be timed and compared.
+
+Four kinds, all through public entry points:
+  layer    the attention block of one layer of a decode step: the new token's
+           rotary embedding, its K/V write and batched paged attention
+           (form "rope"), the write and the attention for callers that rotate
+           elsewhere ("write"), or the attention alone ("plain");
+  prefill  causal attention of new prompt tokens over cached blocks and
+           themselves; with "copy" the new K/V rows are first written into the
+           sequence's blocks, as the runner does for one sequence per layer;
+  step     one batched decode step of the Qwen2.5-0.5B-shaped model through
+           KernelPagedManualDecode (captured graph, projections, norms,
+           attention, head, greedy tokens).
+
+Lengths belong to the case (drawn from its "lens_seed"), so that work() is
+exact; queries, keys, values, block tables, weights and tokens come from the
+seed given to prepare().
+"""
+import math
+import random
+import sys
+from pathlib import Path
+
+import numpy as np
+import torch
+
+sys.path.insert(0, str(Path(__file__).resolve().parent.parent / "vllm-inference-engine_amd"))
+
+from engine import workloads  # noqa: E402
+from engine.kernels.paged_attention import (  # noqa: E402
+    paged_attention_decode_batched,
+    paged_attention_prefill,
+)
+from engine.kernels.paged_attention_integration import (  # noqa: E402
+    KernelPagedManualDecode,
+    paged_decode_kv_write_attention,
+    paged_prefill_copy,
+    paged_rope_decode_attention,
+)
+from engine.memory.block_allocator import BlockTable  # noqa: E402
+
+DEVICE = "cuda"
+ROPE_THETA = 1e6
+MODEL = workloads.QWEN25_05B
+# Every drawn layer or prefill stays within about the listed ones' bytes (the
+# long-context batch) and operations (the fresh prompts).
+MOST_BYTES = 520e6
+MOST_FLOPS = 2.3e11
+
+
+def listed():
+    """The listed cases; heads are query / kv heads, block the tokens of a cache block."""
+    return [
+        # One short conversation: the smallest call a decode step makes per layer.
+        _layer("one short chat", "rope", 1, 14, 2, 64, 16, 300, 300, "equal", 0),
+        # One user with a long document in the context, up to the model's 32768 positions.
+        _layer("one long context", "rope", 1, 14, 2, 64, 16, 24001, 24001, "equal", 0),
+        # A few requests of ragged lengths up to 512: a lightly loaded server.
+        _layer("light load", "write", 8, 14, 2, 64, 16, 1, 512, "uniform", 1),
+        # A few long requests at head_dim 128 (32 / 8 heads): retrieval-augmented prompts.
+        _layer("few long requests", "plain", 8, 32, 8, 128, 16, 1024, 8192, "uniform", 2),
+        # The middle of the batch-128 decode benchmark, one layer.
+        _layer("busy server", "rope", 128, 14, 2, 64, 16, 128, 1088, "uniform", 3),
+        # Equal 2048-token contexts at head_dim 128, 7 query heads per kv head.
+        _layer("equal contexts", "plain", 64, 28, 4, 128, 16, 2048, 2048, "equal", 0),
+        # The headline: 256 requests of ~4.6k tokens, groups of 8 sharing a system prompt.
+        _layer("long contexts, shared prompts", "write", 256, 14, 2, 64, 16, 256, 32768,
+               "lognormal", 4, shared=8),
+        # Eight prompts whose first 2048 tokens are cached, 512 new tokens each.
+        _prefill("cached prompts", 8, 14, 2, 64, 16, 2048, 512, 512, 0, False),
+        # One prompt suffix as the runner prefills it: the K/V copy, then the attention.
+        _prefill("one cached document", 1, 14, 2, 64, 16, 8192, 1001, 1001, 0, True),
+        # A batch of ragged fresh prompts at head_dim 128.
+        _prefill("fresh prompts", 4, 32, 8, 128, 16, 0, 500, 4096, 5, False),
+        # Whole decode steps: a few streams, and the decode benchmark's batch.
+        _step("decode step, 8 streams", 8, 64, 1024, 6),
+        _step("decode step, 128 streams", 128, 64, 1024, 7),
+    ]
+
+
+def _layer(name, form, seqs, heads, kv_heads, dim, block, shortest, longest, spread, lens_seed,
+           shared=0):
+    case = dict(kind="layer", form=form, seqs=seqs, heads=heads, kv_heads=kv_heads, dim=dim,
+                block=block, shortest=shortest, longest=longest, spread=spread,
+                lens_seed=lens_seed, shared=shared)
+    return dict(case, name=name) if name else case
+
+
+def _prefill(name, seqs, heads, kv_heads, dim, block, cached, shortest, longest, lens_seed, copy):
+    case = dict(kind="prefill", seqs=seqs, heads=heads, kv_heads=kv_heads, dim=dim, block=block,
+                cached=cached, shortest=shortest, longest=longest, lens_seed=lens_seed, copy=copy)
+    return dict(case, name=name) if name else case
+
+
+def _step(name, seqs, shortest, longest, lens_seed):
+    case = dict(kind="step", seqs=seqs, shortest=shortest, longest=longest, lens_seed=lens_seed)
+    return dict(case, name=name) if name else case
+
+
+# Head shapes in use: the benchmark model's, common 7-70B-class shapes, and the
+# edges the library is built for (small test models, head_dim 256).
+_HEADS = [(14, 2, 64), (14, 2, 64), (32, 8, 128), (28, 4, 128), (28, 7, 128), (12, 2, 128),
+          (16, 16, 64), (4, 2, 32), (16, 2, 256)]
+
+
+def _log(rng, lo, hi):
+    """A whole number of [lo, hi], spread evenly over its logarithm."""
+    return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    """One more case of the same ranges."""
+    kind = rng.random()
+    lens_seed = rng.randrange(1 << 30)
+    if kind < 0.1:
+        return _step(None, _log(rng, 1, 128), 16, _log(rng, 64, 1024), lens_seed)
+    heads, kv_heads, dim = rng.choice(_HEADS)
+    block = rng.choice([16, 16, 16, 16, 32, 8])
+    while True:
+        if kind < 0.6:
+            seqs = _log(rng, 1, 1280)
+            longest = _log(rng, 16, 32768)
+            spread = rng.choice(["equal", "uniform", "uniform", "lognormal"])
+            shortest = longest if spread == "equal" else rng.randint(1, max(1, longest // 4))
+            shared = rng.choice([0, 0, 0, 8]) if longest > 1024 else 0
+            case = _layer(None, rng.choice(["rope", "write", "plain"]), seqs, heads, kv_heads,
+                          dim, block, shortest, longest, spread, lens_seed, shared)
+        else:
+            seqs = _log(rng, 1, 16)
+            cached = rng.choice([0, _log(rng, 64, 16384) // block * block])
+            longest = _log(rng, 16, 4096)
+            shortest = rng.choice([longest, rng.randint(1, longest)])
+            case = _prefill(None, seqs, heads, kv_heads, dim, block, cached, shortest, longest,
+                            lens_seed, seqs == 1)
+        w = work(case)
+        if w["bytes"] <= MOST_BYTES and w["flops"] <= MOST_FLOPS:
+            return case
+
+
+# ---- lengths and block tables ------------------------------------------------
+
+def _lens(case):
+    """The case's lengths: context lengths (the new token counted), or new prompt tokens."""
+    rng = random.Random(case["lens_seed"])
+    lo, hi, n = case["shortest"], case["longest"], case["seqs"]
+    if case.get("spread") == "equal" or lo == hi:
+        return [hi] * n
+    if case.get("spread") == "lognormal":
+        # Median an eighth of the longest, as 4096 of 32768.
+        return [min(hi, max(lo, int(round(hi / 8 * math.exp(0.5 * rng.gauss(0, 1))))))
+                for _ in range(n)]
+    return [rng.randint(lo, hi) for _ in range(n)]
+
+
+def _shared_blocks(case, lens):
+    """Per sequence, the leading blocks it shares with its group: full blocks, at most 64, never
+    the block of the new token."""
+    if not case.get("shared"):
+        return [0] * len(lens)
+    return [min(64, (n - 1) // case["block"]) for n in lens]
+
+
+def _distinct_slots(case, lens):
+    """Pool rows one attention call reads, a group's shared ones once."""
+    total, size = 0, case.get("shared") or 1
+    shared = _shared_blocks(case, lens)
+    for g in range(0, len(lens), size):
+        group = range(g, min(g + size, len(lens)))
+        total += sum(lens[i] - shared[i] * case["block"] for i in group)
+        total += max(shared[i] for i in group) * case["block"]
+    return total
+
+
+def _tables(case, lens, seed):
+    """(block table rows, pool blocks): ids of a shuffled pool a tenth larger than needed."""
+    bs, size = case["block"], case.get("shared") or 1
+    shared = _shared_blocks(case, lens)
+    need = sum(-(-n // bs) for n in lens)
+    blocks = need + need // 10 + 8
+    ids = np.random.default_rng(seed).permutation(blocks)
+    rows, at = [], 0
+    for g in range(0, len(lens), size):
+        group = range(g, min(g + size, len(lens)))
+        most = max(shared[i] for i in group)
+        prefix, at = ids[at:at + most], at + most
+        for i in group:
+            own = -(-lens[i] // bs) - shared[i]
+            rows.append(np.concatenate([prefix[:shared[i]], ids[at:at + own]]))
+            at += own
+    return rows, blocks
+
+
+def _padded(rows):
+    host = np.zeros((len(rows), max(len(r) for r in rows)), dtype=np.int32)
+    for i, r in enumerate(rows):
+        host[i, :len(r)] = r
+    return torch.from_numpy(host).to(DEVICE)
+
+
+def _normal(shape, gen, std=1.0):
+    return torch.randn(shape, generator=gen, device=DEVICE, dtype=torch.float16).mul_(std)
+
+
+def _int32(values):
+    return torch.tensor(values, dtype=torch.int32, device=DEVICE)
+
+
+def _angles(positions, dim):
+    """Rotary angles of each position, [n, dim], in 64 bits."""
+    inv = ROPE_THETA ** (-torch.arange(0, dim, 2, dtype=torch.float64, device=DEVICE) / dim)
+    a = torch.tensor(positions, dtype=torch.float64, device=DEVICE)[:, None] * inv[None, :]
+    return torch.cat([a, a], dim=1)
+
+
+# ---- prepare -------------------------------------------------------------------
+
+def prepare(case, seed):
+    """What the program holds before the call: pools and tables, and the call's own tensors."""
+    torch.cuda.set_device(0)
+    return {"layer": _prepare_layer, "prefill": _prepare_prefill,
+            "step": _prepare_step}[case["kind"]](case, seed)
+
+
+def _prepare_layer(case, seed):
+    lens = _lens(case)
+    rows, blocks = _tables(case, lens, seed)
+    gen = torch.Generator(device=DEVICE).manual_seed(seed)
+    n, hq, hkv, d = case["seqs"], case["heads"], case["kv_heads"], case["dim"]
+    s = {"case": case, "lens": lens, "rows": rows, "scale": d ** -0.5,
+         "k": _normal((blocks, case["block"], hkv, d), gen),
+         "v": _normal((blocks, case["block"], hkv, d), gen),
+         "tables": _padded(rows), "seq_lens": _int32(lens)}
+    if case["form"] == "rope":
+        # q, k and v as the merged projection leaves them: slices of one buffer.
+        qkv = _normal((n, (hq + 2 * hkv) * d), gen)
+        s["q"] = qkv[:, :hq * d].view(n, hq, d)
+        s["key"] = qkv[:, hq * d:(hq + hkv) * d].view(n, hkv, d)
+        s["value"] = qkv[:, (hq + hkv) * d:].view(n, hkv, d)
+        a = _angles([m - 1 for m in lens], d)
+        s["cos"], s["sin"] = a.cos().half(), a.sin().half()
+    else:
+        s["q"] = _normal((n, hq, d), gen)
+        if case["form"] == "write":
+            s["key"], s["value"] = _normal((n, hkv, d), gen), _normal((n, hkv, d), gen)
+    return s
+
+
+def _prepare_prefill(case, seed):
+    new = _lens(case)
+    total = [case["cached"] + n for n in new]
+    rows, blocks = _tables(case, total, seed)
+    gen = torch.Generator(device=DEVICE).manual_seed(seed)
+    hq, hkv, d, bs = case["heads"], case["kv_heads"], case["dim"], case["block"]
+    start = [0]
+    for n in new:
+        start.append(start[-1] + n)
+    s = {"case": case, "new": new, "lens": total, "rows": rows, "scale": d ** -0.5,
+         "q": _normal((start[-1], hq, d), gen),
+         "k": _normal((blocks, bs, hkv, d), gen), "v": _normal((blocks, bs, hkv, d), gen),
+         "tables": _padded(rows), "seq_lens": _int32(total), "start": _int32(start),
+         "most": max(new)}
+    if case["copy"]:
+        # One sequence's projected rows, [1, kv heads, n, dim] seen as [n, kv heads, dim].
+        s["key"] = _normal((hkv, new[0], d), gen).transpose(0, 1)
+        s["value"] = _normal((hkv, new[0], d), gen).transpose(0, 1)
+        s["write_ids"] = s["tables"][0, case["cached"] // bs:].contiguous()
+    return s
+
+
+def _prepare_step(case, seed):
+    bs = 16
+    lens = _lens(case)
+    rng = np.random.default_rng(seed)
+    need = sum(-(-n // bs) for n in lens)
+    with torch.inference_mode():
+        model = workloads.decode_model(DEVICE, seed=seed)
+        runner = KernelPagedManualDecode(model, num_blocks=need + need // 10 + 8, block_size=bs,
+                                         device=DEVICE)
+        # The streams' cached rows: normal, about as wide as a random projection of a normed row.
+        gen = torch.Generator(device=DEVICE).manual_seed(seed)
+        for cache in runner.pool.k_cache + runner.pool.v_cache:
+            cache.normal_(0.0, 0.6, generator=gen)
+    ids = rng.permutation(runner.num_blocks).tolist()
+    tokens = rng.integers(0, MODEL["vocab_size"], size=len(lens)).tolist()
+    seqs, at = [], 0
+    for i, n in enumerate(lens):
+        own = -(-n // bs)
+        table = BlockTable(seq_id=i, block_size=bs, physical_block_ids=ids[at:at + own],
+                           num_tokens=n - 1)
+        for b in table.physical_block_ids:
+            runner.allocator.ref_counts[b] = 1
+        at += own
+        seqs.append({"seq_id": i, "block_table": table, "last_token_id": tokens[i]})
+    s = {"case": case, "lens": lens, "model": model, "runner": runner, "seqs": seqs}
+    run(s)  # a serving program has captured the batch's graph before
+    return s
+
+
+# ---- run -----------------------------------------------------------------------
+
+def run(s):
+    """One pass; the outputs whole."""
+    kind = s["case"]["kind"]
+    if kind == "layer":
+        form = s["case"]["form"]
+        if form == "rope":
+            out = paged_rope_decode_attention(s["q"], s["key"], s["value"], s["cos"], s["sin"],
+                                              s["k"], s["v"], s["tables"], s["seq_lens"],
+                                              s["scale"])
+        elif form == "write":
+            out = paged_decode_kv_write_attention(s["q"], s["key"], s["value"], s["k"], s["v"],
+                                                  s["tables"], s["seq_lens"], s["scale"])
+        else:
+            return [paged_attention_decode_batched(s["q"], s["k"], s["v"], s["tables"],
+                                                   s["seq_lens"], s["scale"])]
+        return [out, s["k"], s["v"]]
+    if kind == "prefill":
+        if s["case"]["copy"]:
+            paged_prefill_copy(s["key"], s["value"], s["k"], s["v"], s["write_ids"], s["new"][0])
+        out = paged_attention_prefill(s["q"], s["k"], s["v"], s["tables"], s["seq_lens"],
+                                      s["start"], s["most"], s["scale"])
+        return [out, s["k"], s["v"]] if s["case"]["copy"] else [out]
+    # The step counts its token into each stream's table; here every pass is the same step.
+    for seq, n in zip(s["seqs"], s["lens"]):
+        seq["block_table"].num_tokens = n - 1
+    s["runner"].decode_step(s["seqs"])
+    rows = [seq["last_logits"] for seq in s["seqs"]]
+    n, vocab = len(rows), rows[0].shape[0]
+    if rows[-1].data_ptr() - rows[0].data_ptr() == (n - 1) * vocab * rows[0].element_size():
+        return [rows[0].as_strided((n, vocab), (vocab, 1))]  # rows of one buffer
+    return [torch.stack(rows)]
+
+
+# ---- work ----------------------------------------------------------------------
+
+def work(case):
+    """Bytes and operations a pass cannot do without."""
+    lens = _lens(case)
+    if case["kind"] == "layer":
+        hq, hkv, d, n = case["heads"], case["kv_heads"], case["dim"], case["seqs"]
+        nbytes = (4 * hkv * d * _distinct_slots(case, lens) + 4 * n * hq * d
+                  + 4 * sum(-(-m // case["block"]) for m in lens) + 4 * n)
+        if case["form"] != "plain":
+            nbytes += 4 * n * hkv * d  # the pool's new rows written; their source stands for the read
+        if case["form"] == "rope":
+            nbytes += 4 * n * d
+        return {"bytes": nbytes, "flops": 4 * hq * d * sum(lens)}
+    if case["kind"] == "prefill":
+        hq, hkv, d, cached = case["heads"], case["kv_heads"], case["dim"], case["cached"]
+        seen = sum(cached * n + n * (n + 1) // 2 for n in lens)
+        nbytes = 4 * hkv * d * sum(cached + n for n in lens) + 4 * hq * d * sum(lens)
+        if case["copy"]:
+            nbytes += 4 * hkv * d * lens[0]
+        return {"bytes": nbytes, "flops": 4 * hq * d * seen}
+    m = MODEL
+    d = m["hidden_size"] // m["num_attention_heads"]
+    q, kv = m["num_attention_heads"] * d, m["num_key_value_heads"] * d
+    weights = m["num_hidden_layers"] * (m["hidden_size"] * (2 * q + 2 * kv)
+                                        + 3 * m["hidden_size"] * m["intermediate_size"])
+    weights += m["hidden_size"] * m["vocab_size"]
+    return {"bytes": 2 * weights + m["num_hidden_layers"] * 4 * kv * sum(lens)
+            + 2 * case["seqs"] * m["vocab_size"],
+            "flops": 2 * weights * case["seqs"] + m["num_hidden_layers"] * 4 * q * sum(lens)}
+
+
+def tolerance(case):
+    """About four times what another order of the sums shows at these precisions."""
+    if case["kind"] == "layer":
+        # fp16 outputs of fp32 sums: half a unit in the last place each way.
+        return {"rel": 1e-3, "max": 0.01}
+    if case["kind"] == "prefill":
+        # fp16 probabilities too.
+        return {"rel": 2e-3, "max": 0.03}
+    # 24 layers of fp16 activations: a rounding in one travels through all that follow
+    # (the merged projections against the separate ones: 3.7e-3 and 0.021).
+    return {"rel": 1.5e-2, "max": 0.09}
+
+
+# ---- the same in 64 bits ---------------------------------------------------------
+
+def _gather(s, cache, i, n):
+    """The first n rows of sequence i, [kv heads, n, dim] in 64 bits."""
+    ids = torch.from_numpy(np.ascontiguousarray(s["rows"][i])).long().to(DEVICE)
+    rows = cache.index_select(0, ids).flatten(0, 1)[:n]
+    return rows.transpose(0, 1).double().contiguous()
+
+
+def _rotate(x, cos, sin):
+    """Rotary embedding of [..., heads, dim] rows, one angle row each."""
+    half = x.shape[-1] // 2
+    turned = torch.cat([-x[..., half:], x[..., :half]], dim=-1)
+    return x * cos[..., None, :] + turned * sin[..., None, :]
+
+
+def _attend(q, k, v, scale, mask=None):
+    """softmax(scale q k^T) v for q [heads, m, dim], k and v [heads, n, dim]."""
+    scores = torch.bmm(q.contiguous(), k.transpose(1, 2).contiguous()) * scale
+    if mask is not None:
+        scores.masked_fill_(mask, -math.inf)
+    return torch.bmm(torch.softmax(scores, dim=-1), v)
+
+
+def exact(case, seed):
+    """run()'s outputs in 64 bits; None for the pools, which are copies."""
+    return {"layer": _exact_layer, "prefill": _exact_prefill,
+            "step": _exact_step}[case["kind"]](case, seed)
+
+
+def _exact_layer(case, seed):
+    s = _prepare_layer(case, seed)
+    hkv, g = case["kv_heads"], case["heads"] // case["kv_heads"]
+    q = s["q"].double()
+    key = value = None
+    if case["form"] != "plain":
+        key, value = s["key"].double(), s["value"].double()
+    if case["form"] == "rope":
+        cos, sin = s["cos"].double(), s["sin"].double()
+        q, key = _rotate(q, cos, sin), _rotate(key, cos, sin)
+    out = torch.empty(q.shape, dtype=torch.float64, device=DEVICE)
+    for i, n in enumerate(s["lens"]):
+        k, v = _gather(s, s["k"], i, n), _gather(s, s["v"], i, n)
+        if key is not None:
+            k[:, n - 1], v[:, n - 1] = key[i], value[i]
+        out[i] = _attend(q[i].view(hkv, g, -1), k, v, s["scale"]).reshape(q.shape[1:])
+    return [out] if key is None else [out, None, None]
+
+
+def _exact_prefill(case, seed):
+    s = _prepare_prefill(case, seed)
+    hkv, g, d = case["kv_heads"], case["heads"] // case["kv_heads"], case["dim"]
+    out = torch.empty(s["q"].shape, dtype=torch.float64, device=DEVICE)
+    at = 0
+    for i, (new, n) in enumerate(zip(s["new"], s["lens"])):
+        k, v = _gather(s, s["k"], i, n), _gather(s, s["v"], i, n)
+        if case["copy"]:
+            k[:, n - new:] = s["key"].double().transpose(0, 1)
+            v[:, n - new:] = s["value"].double().transpose(0, 1)
+        pos = torch.arange(n - new, n, device=DEVICE).repeat_interleave(g)
+        mask = torch.arange(n, device=DEVICE)[None, :] > pos[:, None]
+        for h in range(hkv):
+            q = s["q"][at:at + new, h * g:(h + 1) * g].double().reshape(1, new * g, d)
+            o = _attend(q, k[h:h + 1], v[h:h + 1], s["scale"], mask[None])
+            out[at:at + new, h * g:(h + 1) * g] = o.view(new, g, d)
+        at += new
+    return [out, None, None] if case["copy"] else [out]
+
+
+@torch.inference_mode()
+def _exact_step(case, seed):
+    s = _prepare_step(case, seed)
+    model, lens, bs = s["model"], s["lens"], 16
+    n, longest = len(lens), max(lens)
+    hq, hkv = MODEL["num_attention_heads"], MODEL["num_key_value_heads"]
+    d = MODEL["hidden_size"] // hq
+    width = -(-longest // bs)
+    ids = torch.zeros(n, width, dtype=torch.long)
+    for i, seq in enumerate(s["seqs"]):
+        row = seq["block_table"].physical_block_ids
+        ids[i, :len(row)] = torch.tensor(row)
+    ids = ids.to(DEVICE)
+    last = torch.tensor(lens, device=DEVICE) - 1
+    streams = torch.arange(n, device=DEVICE)
+    hidden_rows = torch.arange(width * bs, device=DEVICE)[None, :] > last[:, None]
+    mask = hidden_rows[:, None, :].expand(n, hkv, -1).reshape(n * hkv, 1, -1)
+    # The model's own frequencies: a buffer of it, in its precision.
+    angle = last.double()[:, None] * model.model.rotary_emb.inv_freq.double()[None, :]
+    angle = torch.cat([angle, angle], dim=1)
+    cos, sin = angle.cos(), angle.sin()
+
+    def norm(x, module):
+        return (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + module.variance_epsilon)
+                * module.weight.double())
+
+    def linear(x, module):
+        y = x @ module.weight.double().t().contiguous()
+        return y if module.bias is None else y + module.bias.double()
+
+    tokens = torch.tensor([seq["last_token_id"] for seq in s["seqs"]], device=DEVICE)
+    x = model.model.embed_tokens.weight[tokens].double()
+    for i, layer in enumerate(model.model.layers):
+        a, h = layer.self_attn, norm(x, layer.input_layernorm)
+        q = _rotate(linear(h, a.q_proj).view(n, hq, d), cos, sin)
+        key = _rotate(linear(h, a.k_proj).view(n, hkv, d), cos, sin)
+        value = linear(h, a.v_proj).view(n, hkv, d)
+        pool = s["runner"].pool
+        k = pool.k_cache[i][ids].flatten(1, 2).double()
+        v = pool.v_cache[i][ids].flatten(1, 2).double()
+        k[streams, last], v[streams, last] = key, value
+        k = k.transpose(1, 2).reshape(n * hkv, -1, d)
+        v = v.transpose(1, 2).reshape(n * hkv, -1, d)
+        o = _attend(q.view(n * hkv, hq // hkv, d), k, v, d ** -0.5, mask)
+        x = x + linear(o.reshape(n, hq * d), a.o_proj)
+        h, m = norm(x, layer.post_attention_layernorm), layer.mlp
+        gate = linear(h, m.gate_proj)
+        x = x + linear(gate * torch.sigmoid(gate) * linear(h, m.up_proj), m.down_proj)
+    return [linear(norm(x, model.model.norm), model.lm_head)]
