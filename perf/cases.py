@@ -64,7 +64,7 @@ def listed():
         # Equal 2048-token contexts at head_dim 128, 7 query heads per kv head.
         _layer("equal contexts", "plain", 64, 28, 4, 128, 16, 2048, 2048, "equal", 0),
         # The headline: 256 requests of ~4.6k tokens, groups of 8 sharing a system prompt.
-        _layer("long contexts, shared prompts", "write", 256, 14, 2, 64, 16, 256, 32768,
+        _layer("long shared contexts", "write", 256, 14, 2, 64, 16, 256, 32768,
                "lognormal", 4, shared=8),
         # Eight prompts whose first 2048 tokens are cached, 512 new tokens each.
         _prefill("cached prompts", 8, 14, 2, 64, 16, 2048, 512, 512, 0, False),
@@ -73,8 +73,8 @@ def listed():
         # A batch of ragged fresh prompts at head_dim 128.
         _prefill("fresh prompts", 4, 32, 8, 128, 16, 0, 500, 4096, 5, False),
         # Whole decode steps: a few streams, and the decode benchmark's batch.
-        _step("decode step, 8 streams", 8, 64, 1024, 6),
-        _step("decode step, 128 streams", 128, 64, 1024, 7),
+        _step("decode step of 8", 8, 64, 1024, 6),
+        _step("decode step of 128", 128, 64, 1024, 7),
     ]
 
 
