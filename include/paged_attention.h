@@ -57,7 +57,7 @@ enum {
  * with room for shared-prefix records; 12: pa_decode_batched_schedule; 13:
  * pa_decode_kv_write_batched_f16; 14: the decode workspace's head also holds the
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
- * attention launch, 8,448 bytes more). */
+ * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16). */
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */
@@ -366,6 +366,40 @@ PA_API int pa_silu_mul_f16(const void* gate_up, int64_t gate_up_row_stride, void
                            int64_t out_row_stride, int rows, int inter, void* stream);
 PA_API int pa_top2_f16(const void* logits, int64_t row_stride, int rows, int vocab,
                        int64_t* index, float* top, void* stream);
+
+/*
+ * Projections of a decode step's transformer layer over packed operands. No
+ * counterpart in the reference, whose decode step runs transformers' linear
+ * layers (paged_attention_integration.py:620-634 calls the model).
+ *
+ * Packed layout of a [rows, k] fp16 matrix: tiles of 16 rows x 32 columns in
+ * row-tile order (all column tiles of rows 0-15, then of rows 16-31, ...), each
+ * tile 512 consecutive values in the order [column / 8 % 4][row % 16][column %
+ * 8]. Rows are padded to a multiple of 16 (the padding is neither read into a
+ * result nor written); k is a multiple of 32.
+ *
+ * pa_pack_rows_f16: packs row-major rows and writes each row's sum of squares
+ * to row_sums[rows].
+ *
+ * pa_decode_linear_f16: y = epilogue(norm(x) W^T), fp32 accumulation. x is
+ * packed (x_row_stride 0) or row-major; weight [n, k] is packed. With
+ * norm_weight, x (packed) is first RMS-normalised: scaled by norm_weight and by
+ * rsqrt(sum / k + eps), sum being the row's num_row_sums partial sums of
+ * squares row_sums[num_row_sums][rows]. Then bias[n] and the packed residual
+ * [rows, n] are added in fp32 (either may be NULL). With silu_pairs, weight
+ * holds 2 n rows, gate rows then up rows, and y = silu(gate) * up. y is packed
+ * (y_row_stride 0) or row-major fp16, rounded once. row_sums_out, when not
+ * NULL, gets y's partial sums of squares, [n / 16][rows], as the next call's
+ * row_sums.
+ */
+PA_API int pa_pack_rows_f16(const void* x, int64_t x_row_stride, void* packed, float* row_sums,
+                            int rows, int k, void* stream);
+PA_API int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,
+                                const void* norm_weight, const float* row_sums,
+                                int num_row_sums, float eps, const void* bias,
+                                const void* residual, void* y, int64_t y_row_stride,
+                                float* row_sums_out, int rows, int n, int k, int silu_pairs,
+                                void* stream);
 
 /*
  * Batched decode attention that allocates nothing. No counterpart in the

@@ -1,0 +1,142 @@
+"""The decode step's projections over packed operands against fp64 (needs an MI355X).
+
+Bounds. The inputs are fp16, so every product is exact in fp32, and a sum of k
+fp32 terms in any order is within k * 2^-24 of the sum of the terms' absolute
+values; the result is rounded to fp16 once (2^-11 relative). With a norm the
+operand x * scale * weight is itself rounded to fp16 once (2^-11 of each term)
+and the scale is an fp32 rsqrt. SwiGLU's silu adds a few fp32 roundings and its
+derivative (at most 1.1) carries the gate's error.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from engine.kernels.paged_attention_integration import decode_linear, pack_rows, pack_weight
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-6
+
+
+def _data(rows, n, k, device, seed):
+    g = torch.Generator(device=device).manual_seed(seed)
+    x = torch.randn(rows, k, generator=g, device=device).half()
+    w = (torch.randn(n, k, generator=g, device=device) * k ** -0.5).half()
+    return x, w, g
+
+
+def _within(got, want, terms, rel_terms):
+    """|got - want| <= one fp16 rounding + rel_terms of the summed absolute terms."""
+    bound = want.abs() * 2.0 ** -11 + terms * rel_terms + 2.0 ** -24
+    worst = ((got.double() - want).abs() / bound).max().item()
+    print(f"[decode-linear] worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1.0
+
+
+# Row counts at the edges of the 16-row tiles; sizes whose tile counts leave remainders for
+# every tile shape, K from one step (most wavefronts idle) through both wavefront counts.
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 100, 128, 256])
+@pytest.mark.parametrize("n,k", [(32, 32), (1152, 896), (80, 2336), (896, 4864)])
+def test_linear_with_bias_residual_and_sums(cuda_device, rows, n, k):
+    x, w, g = _data(rows, n, k, cuda_device, rows * 31 + n + k)
+    bias = torch.randn(n, generator=g, device=cuda_device).half()
+    want = x.double() @ w.double().t() + bias.double()
+    terms = x.double().abs() @ w.double().abs().t() + bias.double().abs()
+    wp = pack_weight(w)
+    got = decode_linear(x, wp, bias=bias, packed=False)
+    _within(got, want, terms, k * 2.0 ** -24)
+    assert torch.equal(got, decode_linear(pack_rows(x), wp, bias=bias, packed=False))
+    if n % 32:
+        return
+    res = torch.randn(rows, n, generator=g, device=cuda_device).half()
+    out = decode_linear(x, wp, bias=bias, residual=pack_rows(res), sums=True)
+    _within(out.unpack(), want + res.double(), terms + res.double().abs(), (k + 1) * 2.0 ** -24)
+    squares = out.unpack().double().square()
+    assert torch.allclose(out.sums.double().sum(0), squares.sum(1), rtol=n * 2.0 ** -24, atol=0)
+    assert out.sums.shape == (n // 16, rows)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 31, 48, 64, 100, 128, 256])
+@pytest.mark.parametrize("n,k", [(32, 64), (1152, 896), (224, 2304)])
+def test_norm_and_swiglu(cuda_device, rows, n, k):
+    x, w, g = _data(rows, 2 * n, k, cuda_device, rows * 17 + n + k)
+    # Rows of very different sizes: the scale's power of two differs from row to row.
+    x = (x * torch.logspace(-3, 3, rows, device=cuda_device)[:, None]).half()
+    gain = torch.randn(k, generator=g, device=cuda_device).half()
+    xd = x.double()
+    normed = xd * torch.rsqrt(xd.square().mean(1, keepdim=True) + EPS) * gain.double()
+    y = normed @ w.double().t()
+    terms = normed.abs() @ w.double().abs().t()
+    # One rounding of each operand (2^-11), the fp32 scale (a few 2^-24), the sum; operands below
+    # fp16's normal range are rounded to a multiple of 2^-24 of the power-of-two scaled row.
+    rel = 2.0 ** -11 + (k + 8) * 2.0 ** -24
+    small = w.double().abs().sum(1)[None, :] * 2.0 ** -24
+    packed = pack_rows(x)
+    got = decode_linear(packed, pack_weight(w[:n]), norm=(gain, EPS), packed=False)
+    _within(got, y[:, :n], terms[:, :n] + small[:, :n] / rel, rel)
+    act = decode_linear(packed, pack_weight(w), norm=(gain, EPS), silu=True).unpack()
+    gate, up = y[:, :n], y[:, n:]
+    want = torch.nn.functional.silu(gate) * up
+    err = rel * terms + small
+    bound = 1.1 * err[:, :n] * (up.abs() + err[:, n:]) + gate.abs() * err[:, n:]
+    _within(act, want, bound + want.abs() * 2.0 ** -21, 1.0)
+
+
+def test_sums_of_the_previous_launch_feed_the_norm(cuda_device):
+    """A residual row written by one launch is normalised by the next from its partial sums."""
+    x, w, g = _data(37, 896, 896, cuda_device, 3)
+    h = decode_linear(x, pack_weight(w), sums=True)
+    again = pack_rows(h.unpack())
+    assert torch.equal(again.unpack(), h.unpack())
+    gain = torch.rand(896, generator=g, device=cuda_device).half()
+    w2 = pack_weight(_data(1, 1152, 896, cuda_device, 4)[1])
+    a = decode_linear(h, w2, norm=(gain, EPS), packed=False)
+    b = decode_linear(again, w2, norm=(gain, EPS), packed=False)
+    # The row sums differ in order only: the scale by a few 2^-24, the result by an fp16 step.
+    assert ((a.float() - b.float()).abs() <= b.float().abs() * 2.0 ** -10 + 2.0 ** -24).all()
+
+
+def test_rows_with_infinities_and_nans_stay_in_their_rows(cuda_device):
+    x, w, _ = _data(20, 64, 96, cuda_device, 5)
+    x[3, 7], x[18, 0] = float("inf"), float("nan")
+    gain = torch.ones(96, device=cuda_device).half()
+    got = decode_linear(pack_rows(x), pack_weight(w), norm=(gain, EPS), packed=False)
+    bad = torch.zeros(20, dtype=torch.bool, device=cuda_device)
+    bad[[3, 18]] = True
+    assert torch.isnan(got[bad]).all() and torch.isfinite(got[~bad]).all()
+
+
+def test_stack_and_layer_paths_agree(cuda_device):
+    """A decode step through the fused stack, and one that takes the layers one by one (a layer
+    with a forward hook), give the same logits up to fp16 roundings; the hook fires."""
+    from engine import workloads
+    from engine.kernels.paged_attention_integration import KernelPagedManualDecode
+    from engine.memory.block_allocator import BlockTable
+
+    config = dict(vocab_size=512, hidden_size=128, intermediate_size=256, num_hidden_layers=3,
+                  num_attention_heads=4, num_key_value_heads=2, max_position_embeddings=4096,
+                  rope_theta=1e6, tie_word_embeddings=False)
+    with torch.inference_mode():
+        model = workloads.decode_model(cuda_device, 11, config)
+        logits, fired = [], []
+        for hook in (False, True):
+            runner = KernelPagedManualDecode(model, num_blocks=64, device=str(cuda_device),
+                                             use_graphs=False)
+            gen = torch.Generator(device=cuda_device).manual_seed(2)
+            for c in runner.pool.k_cache + runner.pool.v_cache:
+                c.normal_(0, 0.6, generator=gen)
+            seqs = [{"seq_id": i, "block_table": BlockTable(i, 16, [2 * i, 2 * i + 1], 9 + i),
+                     "last_token_id": 5 * i} for i in range(5)]
+            handle = model.model.layers[1].register_forward_hook(
+                lambda *a: fired.append(1)) if hook else None
+            runner.decode_step(seqs)
+            if handle:
+                handle.remove()
+            logits.append(torch.stack([s["last_logits"] for s in seqs]).float())
+    assert fired == [1]
+    # Three layers of fp16 activations: the layer path rounds more often (normed rows, projections
+    # before the residual add); 2^-11 per rounding over some twenty roundings.
+    diff = (logits[0] - logits[1]).norm() / logits[1].norm()
+    print(f"[decode-linear] stack against layers: {diff.item():.2e}", flush=True)
+    assert diff <= 20 * 2.0 ** -11

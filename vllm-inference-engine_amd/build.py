@@ -49,7 +49,11 @@ HIPCC_FLAGS = [
 # copies them out and back, so its MFMAs use the VGPR form. Its score maxima
 # would otherwise quiet possible signalling NaNs with an extra v_max per value
 # (-fno-honor-nans; infinities, which the masking uses, keep their meaning).
+# The decode projections keep their accumulators next to the fragments the same
+# way: in the accumulator-register form each tile would be copied out for the
+# sum over the wavefronts.
 FILE_FLAGS = {
+    "pa_decode_linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "pa_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-fno-honor-nans"],
 }
 

@@ -409,7 +409,7 @@ using namespace pa;
 
 extern "C" {
 
-int pa_abi_version(void) { return 14; }
+int pa_abi_version(void) { return 15; }
 
 const char* pa_last_error(void) { return g_error.c_str(); }
 
@@ -1270,6 +1270,89 @@ int pa_top2_f16(const void* logits, int64_t row_stride, int rows, int vocab, int
   const bool vec = vocab % 8 == 0 && row_stride % 8 == 0 && aligned(logits, 16);
   return finish_launch(launch_top2((const f16*)logits, row_stride, rows, vocab, index, top, vec,
                                    (hipStream_t)stream));
+}
+
+int pa_pack_rows_f16(const void* x, int64_t x_row_stride, void* packed, float* row_sums, int rows,
+                     int k, void* stream) {
+  clear_error();
+  if (rows < 0 || k <= 0 || k % 32) {
+    set_error("rows must be >= 0 and k a positive multiple of 32");
+    return PA_ERR_ARG;
+  }
+  if (rows == 0) return PA_OK;
+  if (!x || !packed || !row_sums) {
+    set_error("null pointer argument");
+    return PA_ERR_ARG;
+  }
+  if (x_row_stride < k || x_row_stride % 8 || !aligned(x, 16) || !aligned(packed, 16) ||
+      !aligned(row_sums, 4)) {
+    set_error("rows need at least k elements, 8-element aligned strides and 16-byte aligned bases");
+    return PA_ERR_ARG;
+  }
+  return finish_launch(launch_pack_rows((const f16*)x, x_row_stride, (f16*)packed, row_sums, rows,
+                                        k, (hipStream_t)stream));
+}
+
+int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,
+                         const void* norm_weight, const float* row_sums, int num_row_sums,
+                         float eps, const void* bias, const void* residual, void* y,
+                         int64_t y_row_stride, float* row_sums_out, int rows, int n, int k,
+                         int silu_pairs, void* stream) {
+  clear_error();
+  if (rows < 0 || n <= 0 || k <= 0 || n % 16 || k % 32) {
+    set_error("rows must be >= 0, n a positive multiple of 16 and k of 32");
+    return PA_ERR_ARG;
+  }
+  if (rows == 0) return PA_OK;
+  if (!x || !weight || !y || (norm_weight && (!row_sums || num_row_sums <= 0))) {
+    set_error("null pointer argument (or a norm without row sums)");
+    return PA_ERR_ARG;
+  }
+  const bool x_packed = x_row_stride == 0, y_packed = y_row_stride == 0;
+  if ((x_row_stride && (x_row_stride < k || x_row_stride % 8)) ||
+      (y_row_stride && (y_row_stride < n || y_row_stride % 4))) {
+    set_error("row-major x rows need at least k elements at an 8-element aligned stride, y rows n "
+              "at a 4-element aligned one (0: packed)");
+    return PA_ERR_ARG;
+  }
+  if ((y_packed || residual) && n % 32) {
+    set_error("a packed output or residual needs n to be a multiple of 32");
+    return PA_ERR_ARG;
+  }
+  if ((norm_weight && !x_packed) || (silu_pairs && (!norm_weight || bias || residual || row_sums_out))) {
+    set_error("norm takes a packed x; silu pairs take a norm and no bias, residual or row sums");
+    return PA_ERR_UNSUPPORTED;
+  }
+  if (!aligned(x, 16) || !aligned(weight, 16) || !aligned(norm_weight, 16) || !aligned(bias, 8) ||
+      !aligned(residual, 8) || !aligned(y, 8) || !aligned(row_sums, 4) || !aligned(row_sums_out, 4)) {
+    set_error("x, weight and norm weight must be 16-byte aligned, bias, residual and y 8-byte");
+    return PA_ERR_ARG;
+  }
+  // Byte offsets inside a tile of rows are 32-bit.
+  if (k > (1 << 25) || x_row_stride > (1 << 24)) {
+    set_error("k %d or the row stride of x exceeds the kernel's 32-bit tile offsets", k);
+    return PA_ERR_UNSUPPORTED;
+  }
+  LinearArgs a{};
+  a.x = (const f16*)x;
+  a.w = (const f16*)weight;
+  a.y = (f16*)y;
+  a.norm = (const f16*)norm_weight;
+  a.ss = row_sums;
+  a.bias = (const f16*)bias;
+  a.res = (const f16*)residual;
+  a.ss_out = row_sums_out;
+  a.ldx = x_row_stride;
+  a.ldy = y_row_stride;
+  a.M = rows;
+  a.N = n;
+  a.K = k;
+  a.ss_parts = num_row_sums;
+  a.y_packed = y_packed;
+  a.inv_k = 1.f / (float)k;
+  a.eps = eps;
+  return finish_launch(launch_decode_linear(a, x_packed, silu_pairs != 0, device_cus(),
+                                            (hipStream_t)stream));
 }
 
 }  // extern "C"

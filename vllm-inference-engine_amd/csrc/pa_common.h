@@ -338,4 +338,35 @@ __device__ inline int num_splits_for(int ntiles, int split_tiles) {
 // 16 denominators, then 16 x D unnormalised accumulators (row = q head in group).
 __host__ __device__ constexpr int record_floats(int D) { return 32 + 16 * D; }
 
+// Argument bundle of the decode step's projections: y[m, n] = sum_k x[m, k]
+// w[n, k] over the packed layout below.
+struct LinearArgs {
+  const f16* x;    // [M, K] packed, or row-major with row stride ldx
+  const f16* w;    // [N, K] packed (with silu [2 N, K]: gate rows, then up rows)
+  f16* y;          // [M, N] packed, or row-major with row stride ldy
+  const f16* norm;  // RMSNorm weight [K] applied to x, or null
+  const float* ss;  // with norm: ss_parts partial sums of squares per row, [ss_parts][M]
+  const f16* bias;  // [N] or null
+  const f16* res;   // [M, N] packed, added to the product, or null
+  float* ss_out;    // per 16-column tile of y its rows' sums of squares, [N / 16][M], or null
+  int64_t ldx, ldy;
+  int M, N, K;
+  int mtiles;  // workgroups along M (set at launch)
+  int ss_parts, y_packed;
+  float inv_k, eps;
+};
+
+// Packed layout of a [rows, K] operand: 16-row x 32-column tiles in row-tile
+// order, each 512 consecutive values in the lane order of a 16x16x32 MFMA
+// operand (lane 16 (k % 32 / 8) + row % 16 holds 8 consecutive k).
+__host__ __device__ inline int64_t pack_index(int row, int k, int K) {
+  return ((int64_t)(row >> 4) * (K / 32) + (k >> 5)) * 512 + ((k & 31) >> 3) * 128 +
+         (row & 15) * 8 + (k & 7);
+}
+
+hipError_t launch_decode_linear(const LinearArgs& a, bool x_packed, bool silu, int cus,
+                                hipStream_t s);
+hipError_t launch_pack_rows(const f16* x, int64_t ldx, f16* y, float* ss, int rows, int K,
+                            hipStream_t s);
+
 }  // namespace pa

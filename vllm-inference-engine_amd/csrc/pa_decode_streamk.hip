@@ -43,14 +43,6 @@ namespace pa {
 
 using namespace tiles;
 
-// Position of workgroup i among n in an order in which each XCD (workgroup i
-// runs on XCD i % 8) owns a contiguous run of positions.
-__device__ inline int xcd_order(int i, int n) {
-  const int n8 = n / kXcds, rem = n % kXcds;
-  const int xcd = i % kXcds, k = i / kXcds;
-  return xcd * n8 + (xcd < rem ? xcd : rem) + k;
-}
-
 // A wavefront-uniform value, moved to a scalar register.
 __device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 

@@ -9,6 +9,14 @@ namespace tiles {
 
 constexpr int kXcds = 8;  // accelerator complex dies of an MI355X, each with its own L2
 
+// Position of workgroup i among n in an order in which each XCD (workgroup i
+// runs on XCD i % 8) owns a contiguous run of positions.
+__device__ inline int xcd_order(int i, int n) {
+  const int n8 = n / kXcds, rem = n % kXcds;
+  const int xcd = i % kXcds, k = i / kXcds;
+  return xcd * n8 + (xcd < rem ? xcd : rem) + k;
+}
+
 __device__ inline f16x8 zero8() { return f16x8{0, 0, 0, 0, 0, 0, 0, 0}; }
 
 // K/V register buffers hold raw 16-byte pieces as 32-bit lanes: kept as fp16

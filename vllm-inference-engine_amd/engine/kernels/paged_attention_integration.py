@@ -61,6 +61,11 @@ __all__ = [
     "rms_norm",
     "silu_mul",
     "greedy_top2",
+    "fused_decoder_stack_forward",
+    "pack_weight",
+    "pack_rows",
+    "PackedRows",
+    "decode_linear",
     "KernelPagedManualDecode",
 ]
 
@@ -617,6 +622,122 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+# ---- the decode step's projections over packed operands -------------------------
+
+# Rows up to which a decode step's projections take pa_decode_linear_f16: a layer's
+# four launches against the library GEMMs with their norm and SwiGLU launches,
+# measured in captured graphs on the 0.5B-class model: 128 rows 27 against 59 us,
+# 256 rows 39 against about 53; at 512 rows 67 against 62.
+DECODE_LINEAR_MAX_ROWS = 256
+
+
+def _packable(weight: torch.Tensor) -> bool:
+    return (weight.dim() == 2 and weight.dtype == torch.float16 and weight.shape[0] % 16 == 0
+            and weight.shape[1] % 32 == 0)
+
+
+def pack_weight(weight: torch.Tensor) -> torch.Tensor:
+    """An fp16 [n, k] weight (n % 16 == 0, k % 32 == 0) in the packed layout pa_decode_linear_f16 reads.
+
+    Tiles of 16 rows x 32 columns, each in the order [column / 8][row][column % 8].
+    """
+    assert _packable(weight)
+    n, k = weight.shape
+    return weight.reshape(n // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
+
+
+class PackedRows:
+    """fp16 rows [rows, width] in the packed layout, with each row's partial sums of squares."""
+
+    __slots__ = ("data", "rows", "width", "sums")
+
+    def __init__(self, rows: int, width: int, parts: int, device: torch.device):
+        assert width % 32 == 0
+        self.rows, self.width = rows, width
+        self.data = torch.empty(-(-rows // 16) * 16 * width, dtype=torch.float16, device=device)
+        self.sums = torch.empty(parts, rows, dtype=torch.float32, device=device) if parts else None
+
+    def unpack(self) -> torch.Tensor:
+        """The rows, row-major."""
+        t = self.data.view(-1, self.width // 32, 4, 16, 8).permute(0, 3, 1, 2, 4)
+        return t.reshape(-1, self.width)[:self.rows]
+
+
+def pack_rows(x: torch.Tensor) -> PackedRows:
+    """Row-major fp16 rows [rows, k] to the packed layout, with their sums of squares."""
+    assert x.is_cuda and x.dtype == torch.float16 and x.dim() == 2
+    x = _rows16(x)
+    rows, k = x.shape
+    out = PackedRows(rows, k, 1, x.device)
+    lib = _native.load()
+    with _on_device(x.device):
+        status = lib.pa_pack_rows_f16(x.data_ptr(), x.stride(0), out.data.data_ptr(),
+                                      out.sums.data_ptr(), rows, k,
+                                      _native.stream_handle(x.device))
+    _native.check(status, "pa_pack_rows_f16")
+    return out
+
+
+def decode_linear(
+    x: Union[torch.Tensor, PackedRows],  # rows [rows, k]
+    weight: torch.Tensor,                # pack_weight of [n, k]; with silu of [2 n, k] (gate, up)
+    norm: Optional[Tuple[torch.Tensor, float]] = None,  # RMSNorm weight [k] and eps, for a packed x
+    bias: Optional[torch.Tensor] = None,
+    residual: Optional[PackedRows] = None,
+    silu: bool = False,
+    packed: bool = True,
+    sums: bool = False,
+) -> Union[torch.Tensor, PackedRows]:
+    """norm(x) W^T + bias + residual, or silu(gate) * up, in one launch (fp32 sums, rounded once).
+
+    Returns PackedRows (with the partial sums of squares a following norm needs,
+    if asked) or, with packed=False, a row-major [rows, n] tensor.
+    """
+    k = weight.shape[1] * 32
+    n = weight.shape[0] * 16 // (2 if silu else 1)
+    if isinstance(x, PackedRows):
+        xd, x_stride, rows, width = x.data, 0, x.rows, x.width
+    else:
+        x = _rows16(x)
+        xd, x_stride, (rows, width) = x, x.stride(0), x.shape
+    assert xd.is_cuda and xd.dtype == torch.float16 and weight.dtype == torch.float16
+    assert width == k, f"x rows of {width} values do not match the weight's {k}"
+    ptrs = [0, 0, 0, 0, 0]  # norm weight, row sums, bias, residual, row sums out
+    parts, eps = 0, 0.0
+    same = [xd, weight]
+    if norm is not None:
+        assert isinstance(x, PackedRows) and x.sums is not None
+        w, eps = norm
+        assert w.dtype == torch.float16 and w.shape == (k,) and w.is_contiguous()
+        ptrs[0], ptrs[1], parts = w.data_ptr(), x.sums.data_ptr(), x.sums.shape[0]
+        same.append(w)
+    if bias is not None:
+        assert bias.dtype == torch.float16 and bias.shape == (n,) and bias.is_contiguous()
+        ptrs[2] = bias.data_ptr()
+        same.append(bias)
+    if residual is not None:
+        assert (residual.rows, residual.width) == (rows, n)
+        ptrs[3] = residual.data.data_ptr()
+        same.append(residual.data)
+    _native.same_device(*same)
+    if packed:
+        out = PackedRows(rows, n, n // 16 if sums else 0, xd.device)
+        y_ptr, y_stride = out.data.data_ptr(), 0
+        if sums:
+            ptrs[4] = out.sums.data_ptr()
+    else:
+        out = torch.empty(rows, n, dtype=torch.float16, device=xd.device)
+        y_ptr, y_stride = out.data_ptr(), n
+    lib = _native.load()
+    with _on_device(xd.device):
+        status = lib.pa_decode_linear_f16(
+            xd.data_ptr(), x_stride, weight.data_ptr(), ptrs[0], ptrs[1], parts, float(eps), ptrs[2],
+            ptrs[3], y_ptr, y_stride, ptrs[4], rows, n, k, int(silu),
+            _native.stream_handle(xd.device))
+    _native.check(status, "pa_decode_linear_f16")
+    return out
+
+
 def _is_decoder_layer(m: nn.Module) -> bool:
     attn, mlp = getattr(m, "self_attn", None), getattr(m, "mlp", None)
     return (attn is not None and mlp is not None
@@ -629,8 +750,11 @@ def prepare_fused_layers(model: nn.Module) -> int:
     """Concatenate each decoder layer's q/k/v and gate/up weights once, for the fused decode path.
 
     The merged copies live on the layer (`_pa_fused`); the model's own modules
-    are left as they are. Returns the number of layers prepared. Inference
-    only: the copies do not follow later changes of the weights.
+    are left as they are. Where the sizes allow it, all four projections are
+    also kept in the packed layout of the decode-step kernels (`_pa_packed`:
+    q/k/v, o, gate/up, down; fused_decoder_stack_forward). Returns the number of
+    layers prepared. Inference only: the copies do not follow later changes of
+    the weights.
     """
     n = 0
     if not isinstance(model, nn.Module):
@@ -652,6 +776,10 @@ def prepare_fused_layers(model: nn.Module) -> int:
                 qkv_b,
                 torch.cat([mlp.gate_proj.weight, mlp.up_proj.weight]).contiguous(),
             )
+            weights = (m._pa_fused[0], attn.o_proj.weight, m._pa_fused[2], mlp.down_proj.weight)
+            if all(w.is_cuda and _packable(w) for w in weights) and \
+                    weights[0].shape[1] % 32 == 0 and weights[3].shape[0] % 32 == 0:
+                m._pa_packed = tuple(pack_weight(w) for w in weights)
             n += 1
     return n
 
@@ -714,6 +842,82 @@ def fused_decoder_layer_forward(
     return h.view(b, 1, hidden)
 
 
+def _has_hooks(m: nn.Module) -> bool:
+    return bool(m._forward_hooks or m._forward_pre_hooks)
+
+
+def _stack_takes(self: nn.Module, input_ids, attention_mask, position_ids, past_key_values,
+                 inputs_embeds, use_cache, kwargs) -> bool:
+    """Whether a call of the base model is a plain decode step the fused stack computes whole."""
+    ctx = self._paged_stack_context
+    from torch.nn.modules import module as _module
+
+    return (ctx is not None and ctx.is_decode and ctx.is_batched
+            and input_ids is not None and input_ids.dim() == 2 and input_ids.shape[1] == 1
+            and 0 < input_ids.shape[0] <= DECODE_LINEAR_MAX_ROWS
+            and attention_mask is None and position_ids is not None and past_key_values is None
+            and inputs_embeds is None and not use_cache and not any(kwargs.values())
+            and not getattr(self.config, "output_hidden_states", False)
+            and not getattr(self.config, "output_attentions", False)
+            and not _module._global_forward_hooks and not _module._global_forward_pre_hooks
+            and not any(_has_hooks(layer) for layer in self.layers))
+
+
+def fused_decoder_stack_forward(
+    self: nn.Module,
+    input_ids: Optional[torch.Tensor] = None,
+    attention_mask: Optional[torch.Tensor] = None,
+    position_ids: Optional[torch.Tensor] = None,
+    past_key_values: Any = None,
+    inputs_embeds: Optional[torch.Tensor] = None,
+    use_cache: Optional[bool] = None,
+    **kwargs: Any,
+) -> Any:
+    """transformers' Qwen2Model.forward for one decode step, five launches per decoder layer.
+
+    The computation of the layers patched with fused_decoder_layer_forward, with
+    the residual stream kept packed between the launches: input norm + q/k/v;
+    RoPE, K/V write and paged attention; o + residual; post-attention norm +
+    gate/up + SwiGLU; down + residual. Calls that ask for more than a decode
+    step's hidden states (masks, caches, hidden-state outputs), layers with
+    forward hooks and more than DECODE_LINEAR_MAX_ROWS rows take the layers one
+    by one as before.
+    """
+    if not _stack_takes(self, input_ids, attention_mask, position_ids, past_key_values,
+                        inputs_embeds, use_cache, kwargs):
+        return self._orig_stack_forward(input_ids=input_ids, attention_mask=attention_mask,
+                                        position_ids=position_ids, past_key_values=past_key_values,
+                                        inputs_embeds=inputs_embeds, use_cache=use_cache, **kwargs)
+    from transformers.modeling_outputs import BaseModelOutputWithPast
+
+    ctx = self._paged_stack_context
+    x = self.embed_tokens(input_ids)
+    b, _, hidden = x.shape
+    cos, sin = self.rotary_emb(x, position_ids)
+    rows = pack_rows(x.view(b, hidden))
+    layers = self.layers[:self.config.num_hidden_layers]
+    for i, layer in enumerate(layers):
+        attn, mlp = layer.self_attn, layer.mlp
+        qkv_w, o_w, gu_w, down_w = layer._pa_packed
+        hd = attn.head_dim
+        nq = attn.q_proj.out_features // hd
+        nkv = attn.k_proj.out_features // hd
+        norm1, norm2 = layer.input_layernorm, layer.post_attention_layernorm
+        qkv = decode_linear(rows, qkv_w, norm=(norm1.weight, norm1.variance_epsilon),
+                            bias=layer._pa_fused[1], packed=False)
+        scale = attn.scaling if hasattr(attn, "scaling") else 1.0 / math.sqrt(hd)
+        o = paged_rope_decode_attention(
+            qkv[:, :nq * hd].view(b, nq, hd), qkv[:, nq * hd:(nq + nkv) * hd].view(b, nkv, hd),
+            qkv[:, (nq + nkv) * hd:].view(b, nkv, hd), cos, sin, ctx.pool.k_cache[attn.layer_idx],
+            ctx.pool.v_cache[attn.layer_idx], ctx.padded_block_tables, ctx.seq_lens_tensor, scale)
+        h = decode_linear(o.view(b, nq * hd), o_w, bias=attn.o_proj.bias, residual=rows, sums=True)
+        act = decode_linear(h, gu_w, norm=(norm2.weight, norm2.variance_epsilon), silu=True)
+        last = i + 1 == len(layers)
+        rows = decode_linear(act, down_w, residual=h, packed=not last, sums=not last)
+    x = rows if layers else x
+    return BaseModelOutputWithPast(last_hidden_state=self.norm(x.view(b, 1, hidden)))
+
+
 def _fused_rms_norm_forward(self: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:
     if hidden_states.dtype != torch.float16 or self.weight.dtype != torch.float16:
         return self._orig_norm_forward(hidden_states)
@@ -746,6 +950,13 @@ def patch_paged_attention(model: nn.Module, context: PagedAttentionContext,
             module._orig_layer_forward = orig_fwd
             module.forward = fused_decoder_layer_forward.__get__(module, module.__class__)
             patched.append((module, orig_fwd, "layer"))
+        elif decode and type(module).__name__ == "Qwen2Model" and \
+                all(hasattr(layer, "_pa_packed") for layer in module.layers):
+            orig_fwd = module.forward
+            module._orig_stack_forward = orig_fwd
+            module._paged_stack_context = context
+            module.forward = fused_decoder_stack_forward.__get__(module, module.__class__)
+            patched.append((module, orig_fwd, "stack"))
     if any(kind == "layer" for _, _, kind in patched):
         for module in model.modules():
             if hasattr(module, "variance_epsilon") and isinstance(getattr(module, "weight", None),
@@ -767,7 +978,8 @@ def patch_paged_attention(model: nn.Module, context: PagedAttentionContext,
             else:
                 module.forward = orig_fwd
             for attr in ("_orig_attention_forward", "_paged_attention_context",
-                         "_orig_layer_forward", "_orig_norm_forward"):
+                         "_orig_layer_forward", "_orig_norm_forward", "_orig_stack_forward",
+                         "_paged_stack_context"):
                 if hasattr(module, attr):
                     delattr(module, attr)
 
