@@ -247,3 +247,25 @@ def test_prefill_and_decode_interleaved_on_one_stream(cuda_device):
         assert torch.equal(run(c, 0.125), p0)
         assert torch.equal(paged_attention_decode_batched(d["qd"], d["kd"], d["vd"], d["btd"],
                                                           d["lensd"], 0.125), d0)
+
+
+# Ragged batches number their workgroups over the column blocks that exist, up to 256 sequences
+# (four per lane) and over every sequence's longest beyond: edges of the lane groups, sequences
+# without new tokens first, last and between, a column block filled exactly and by one column.
+@pytest.mark.parametrize("num_seqs", [2, 3, 63, 64, 65, 130, 256, 257])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 2, 32), (16, 2, 128)])
+def test_ragged_batches(cuda_device, num_seqs, hq, hkv, d):
+    rnd = random.Random(num_seqs * d)
+    g, cols = hq // hkv, 128
+    new = [rnd.choice([0, 1, 3, 16, cols // g, cols // g + 1, 70]) for _ in range(num_seqs)]
+    new[0], new[-1] = 0, 2 * cols // g
+    if num_seqs > 4:
+        new[1], new[-2] = 5 * cols // g + 1, 0
+    ctx = [max(1, n + rnd.choice([0, 0, 5, 40])) for n in new]
+    c = build(hq, hkv, d, 16, ctx, new, seed=num_seqs, device=cuda_device, slack=1)
+    scale = d ** -0.5
+    out = run(c, scale)
+    assert torch.isfinite(out).all()
+    err = max_err(out, oracle(c, scale))
+    print(f"[prefill] ragged {num_seqs} seqs d={d} max_err={err:.2e}", flush=True)
+    assert err <= TOL

@@ -1195,6 +1195,12 @@ int pa_prefill_attention_f16(const void* q, const int64_t q_strides[3], const vo
   a.scale_log2 = scale * kLog2e;
   a.split_tiles = (int)plan.split_tiles;
   a.max_splits = (int)plan.max_splits;
+  // Batches whose sequences are not all max_query_len long: at most one partly
+  // filled column block per sequence beside the full ones.
+  const int cols = 64 * plan.col_groups;
+  const int64_t exist = (int64_t)num_tokens * g / cols + num_seqs;
+  if (num_seqs > 1 && num_seqs <= kPfCompactSeqs && exist < plan.col_blocks * num_seqs)
+    a.compact = (int)exist;
   a.cnt = plan.ws_bytes ? (int*)workspace : nullptr;
   a.recs = plan.ws_bytes ? (float*)((char*)workspace + plan.counter_bytes) : nullptr;
   return finish_launch(launch_prefill_attn(a, head_dim, (hipStream_t)stream));

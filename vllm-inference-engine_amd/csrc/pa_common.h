@@ -221,6 +221,10 @@ struct PrefillAttnArgs {
   // tiles is processed by several workgroups (up to max_splits), which leave
   // partial records; the last to finish merges them.
   int split_tiles, max_splits;
+  // Ragged batches of up to kPfCompactSeqs sequences: the column blocks that can
+  // exist (an upper bound from num_tokens), over which the workgroups are
+  // numbered; 0: numbered over col_blocks per sequence.
+  int compact;
   int* cnt;     // per-column-block arrival counters, zero between launches
   float* recs;  // [seq][kv head][column block][split] records of (D + 2) x columns floats
 };
@@ -232,6 +236,9 @@ struct PrefillAttnArgs {
 // or eight wavefronts of one group, chosen per launch by prefill_plan. Launches
 // with few column blocks take one unit instead (twice the workgroups).
 __host__ __device__ constexpr int prefill_col_groups(int D) { return D <= 128 ? 2 : 1; }
+// Sequences of a ragged prefill batch whose workgroups are numbered over the
+// column blocks that exist (four per lane of a wavefront).
+constexpr int kPfCompactSeqs = 256;
 // The prefill workspace starts with a fixed region of arrival counters, one per
 // column block of a split launch, so that the counters of every launch sit at
 // the same place whatever its size and never overlap an earlier launch's

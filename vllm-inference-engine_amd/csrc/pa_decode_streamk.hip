@@ -65,19 +65,6 @@ __host__ __device__ inline int64_t range_start(int w, int64_t T, int G) {
   return (int64_t)w * T / G;
 }
 
-// Inclusive prefix sum over the 64 lanes of a wavefront in DPP lane moves:
-// shifts by 1, 2, 4 and 8 within each row of 16 lanes (zero shifted in), then
-// each row's total broadcast to the rows after it (row_bcast 15 and 31).
-__device__ inline int wave_incl_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 (rows 1, 3)
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 (rows 2, 3)
-  return x;
-}
-
 // Exclusive prefix sums over a workgroup of NW wavefronts, PER values per
 // thread (thread t holds entries t * PER .. t * PER + PER - 1); returns the
 // total. s_tot holds NW ints, written once per call with one barrier: a
