@@ -57,7 +57,8 @@ enum {
  * with room for shared-prefix records; 12: pa_decode_batched_schedule; 13:
  * pa_decode_kv_write_batched_f16; 14: the decode workspace's head also holds the
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
- * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16). */
+ * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
+ * 16: pa_decode_embed_f16). */
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */
@@ -391,9 +392,20 @@ PA_API int pa_top2_f16(const void* logits, int64_t row_stride, int rows, int voc
  * (y_row_stride 0) or row-major fp16, rounded once. row_sums_out, when not
  * NULL, gets y's partial sums of squares, [n / 16][rows], as the next call's
  * row_sums.
+ *
+ * pa_decode_embed_f16: the start of a decode step: row r of packed is the fp16
+ * embedding row table[ids[r]] (NaNs for an id outside [0, vocab)), row_sums[r]
+ * its sum of squares, and cos / sin [rows, head_dim] the fp16 rotary rows of
+ * positions[r]: cos(inv_freq[j] * position) * scaling in fp32 for j <
+ * head_dim / 2, repeated in the second half (Qwen2RotaryEmbedding.forward);
+ * inv_freq is fp32, or fp16 with inv_freq_half.
  */
 PA_API int pa_pack_rows_f16(const void* x, int64_t x_row_stride, void* packed, float* row_sums,
                             int rows, int k, void* stream);
+PA_API int pa_decode_embed_f16(const int64_t* ids, const int64_t* positions, const void* table,
+                               int64_t vocab, int hidden, const void* inv_freq, int inv_freq_half,
+                               float scaling, int head_dim, void* packed, float* row_sums,
+                               void* cos, void* sin, int rows, void* stream);
 PA_API int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,
                                 const void* norm_weight, const float* row_sums,
                                 int num_row_sums, float eps, const void* bias,

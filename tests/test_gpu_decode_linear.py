@@ -140,3 +140,31 @@ def test_stack_and_layer_paths_agree(cuda_device):
     diff = (logits[0] - logits[1]).norm() / logits[1].norm()
     print(f"[decode-linear] stack against layers: {diff.item():.2e}", flush=True)
     assert diff <= 20 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("rows,hidden,dim,freq", [
+    (1, 32, 64, torch.float32), (17, 896, 64, torch.float16), (130, 2336, 128, torch.float32)])
+def test_embed_matches_the_modules(cuda_device, rows, hidden, dim, freq):
+    """Embedding rows bit for bit; cos and sin as torch computes them in fp32 (an fp16 rounding
+    boundary apart at most); an id outside the table gives NaNs in its row only."""
+    from engine.kernels.paged_attention_integration import decode_embed
+
+    g = torch.Generator(device=cuda_device).manual_seed(rows)
+    table = torch.randn(1000, hidden, generator=g, device=cuda_device).half()
+    ids = torch.randint(0, 1000, (rows,), generator=g, device=cuda_device)
+    pos = torch.randint(0, 32768, (rows,), generator=g, device=cuda_device)
+    inv = 1e6 ** (-torch.arange(0, dim, 2, device=cuda_device).float() / dim)
+    inv = inv.to(freq)
+    packed, cos, sin = decode_embed(ids, pos, table, inv, 0.5)
+    assert torch.equal(packed.unpack(), table[ids])
+    assert torch.allclose(packed.sums[0].double(), table[ids].double().square().sum(1),
+                          rtol=hidden * 2.0 ** -24, atol=0)
+    angle = (pos.float()[:, None] * inv.float()[None, :]).repeat(1, 2)
+    for got, want in ((cos, angle.cos() * 0.5), (sin, angle.sin() * 0.5)):
+        assert ((got.float() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -22).all()
+    if rows > 1:
+        ids[1], ids[-1] = -1, 1000
+        out = decode_embed(ids, pos, table, inv)[0].unpack()
+        bad = torch.zeros(rows, dtype=torch.bool, device=cuda_device)
+        bad[[1, rows - 1]] = True
+        assert torch.isnan(out[bad]).all() and torch.equal(out[~bad], table[ids[~bad]])

@@ -409,7 +409,7 @@ using namespace pa;
 
 extern "C" {
 
-int pa_abi_version(void) { return 15; }
+int pa_abi_version(void) { return 16; }
 
 const char* pa_last_error(void) { return g_error.c_str(); }
 
@@ -1297,6 +1297,43 @@ int pa_pack_rows_f16(const void* x, int64_t x_row_stride, void* packed, float* r
   }
   return finish_launch(launch_pack_rows((const f16*)x, x_row_stride, (f16*)packed, row_sums, rows,
                                         k, (hipStream_t)stream));
+}
+
+int pa_decode_embed_f16(const int64_t* ids, const int64_t* positions, const void* table,
+                        int64_t vocab, int hidden, const void* inv_freq, int inv_freq_half,
+                        float scaling, int head_dim, void* packed, float* row_sums, void* cos,
+                        void* sin, int rows, void* stream) {
+  clear_error();
+  if (rows < 0 || vocab <= 0 || hidden <= 0 || hidden % 32 || head_dim <= 0 || head_dim % 2) {
+    set_error("rows must be >= 0, vocab positive, hidden a positive multiple of 32 and head_dim a "
+              "positive even number");
+    return PA_ERR_ARG;
+  }
+  if (rows == 0) return PA_OK;
+  if (!ids || !positions || !table || !inv_freq || !packed || !row_sums || !cos || !sin) {
+    set_error("null pointer argument");
+    return PA_ERR_ARG;
+  }
+  if (!aligned(ids, 8) || !aligned(positions, 8) || !aligned(table, 16) || !aligned(packed, 16) ||
+      !aligned(inv_freq, inv_freq_half ? 2 : 4) || !aligned(row_sums, 4) || !aligned(cos, 2) || !aligned(sin, 2)) {
+    set_error("table and packed rows must be 16-byte aligned, the others naturally");
+    return PA_ERR_ARG;
+  }
+  DecodeEmbedArgs a{};
+  a.ids = ids;
+  a.pos = positions;
+  a.table = (const f16*)table;
+  a.inv_freq = inv_freq_half ? nullptr : (const float*)inv_freq;
+  a.inv_freq_half = (const f16*)inv_freq;
+  a.x = (f16*)packed;
+  a.ss = row_sums;
+  a.cos = (f16*)cos;
+  a.sin = (f16*)sin;
+  a.vocab = vocab;
+  a.H = hidden;
+  a.dim = head_dim;
+  a.scaling = scaling;
+  return finish_launch(launch_decode_embed(a, rows, (hipStream_t)stream));
 }
 
 int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,

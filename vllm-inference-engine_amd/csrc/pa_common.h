@@ -373,6 +373,22 @@ __host__ __device__ inline int64_t pack_index(int row, int k, int K) {
 
 hipError_t launch_decode_linear(const LinearArgs& a, bool x_packed, bool silu, int cus,
                                 hipStream_t s);
+// Argument bundle of a decode step's start: embedding rows and rotary rows.
+struct DecodeEmbedArgs {
+  const int64_t* ids;
+  const int64_t* pos;
+  const f16* table;  // [vocab, H]
+  const float* inv_freq;     // [dim / 2], or null:
+  const f16* inv_freq_half;  // the same in fp16
+  f16* x;     // [rows, H] packed
+  float* ss;  // [rows]
+  f16* cos;   // [rows, dim]
+  f16* sin;
+  int64_t vocab;
+  int H, dim;
+  float scaling;
+};
+hipError_t launch_decode_embed(const DecodeEmbedArgs& a, int rows, hipStream_t s);
 hipError_t launch_pack_rows(const f16* x, int64_t ldx, f16* y, float* ss, int rows, int K,
                             hipStream_t s);
 

@@ -208,6 +208,50 @@ __global__ __launch_bounds__(1024) void top2_kernel(const f16* __restrict__ logi
   }
 }
 
+// The start of a decode step, one workgroup per row: the token's embedding row
+// into the packed layout with its sum of squares, and its rotary cos and sin
+// rows (modeling_qwen2.Qwen2RotaryEmbedding.forward: fp32 angle inv_freq *
+// position, inv_freq a buffer in the model's precision, cos and sin in fp32 times the scaling, rounded to fp16; the second
+// half of a row repeats the first). As torch ops these are about a dozen
+// launches of 2-4 us each on a few KB. A token id outside the table gives a row
+// of NaNs.
+__global__ __launch_bounds__(256) void decode_embed_kernel(DecodeEmbedArgs a) {
+  const int m = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int64_t id = a.ids[m];
+  const float pos = (float)a.pos[m];
+  const bool known = id >= 0 && id < a.vocab;
+  const f16* row = a.table + (known ? id : 0) * a.H;
+  float s = 0.f;
+  for (int k = tid * 8; k < a.H; k += 256 * 8) {
+    f16x8 v = *reinterpret_cast<const f16x8*>(row + k);
+    if (!known) v = f16x8(__builtin_nanf(""));
+    *reinterpret_cast<f16x8*>(a.x + pack_index(m, k, a.H)) = v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)v[e], (float)v[e], s);
+  }
+  const int half = a.dim / 2;
+  for (int j = tid; j < half; j += 256) {
+    const float angle = (a.inv_freq ? a.inv_freq[j] : (float)a.inv_freq_half[j]) * pos;
+    const f16 c = (f16)(cosf(angle) * a.scaling), n = (f16)(sinf(angle) * a.scaling);
+    a.cos[(int64_t)m * a.dim + j] = c;
+    a.cos[(int64_t)m * a.dim + half + j] = c;
+    a.sin[(int64_t)m * a.dim + j] = n;
+    a.sin[(int64_t)m * a.dim + half + j] = n;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  __shared__ float part[4];
+  if ((tid & 63) == 0) part[tid >> 6] = s;
+  __syncthreads();
+  if (tid == 0) a.ss[m] = part[0] + part[1] + part[2] + part[3];
+}
+
+hipError_t launch_decode_embed(const DecodeEmbedArgs& a, int rows, hipStream_t s) {
+  decode_embed_kernel<<<rows, 256, 0, s>>>(a);
+  return hipGetLastError();
+}
+
 hipError_t launch_rmsnorm(const f16* x, int64_t xs, const f16* res, int64_t rs, f16* sum,
                           int64_t ss, const f16* w, f16* y, int64_t ys, int rows, int H,
                           float eps, hipStream_t s) {

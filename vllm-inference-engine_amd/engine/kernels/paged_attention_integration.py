@@ -66,6 +66,7 @@ __all__ = [
     "pack_rows",
     "PackedRows",
     "decode_linear",
+    "decode_embed",
     "KernelPagedManualDecode",
 ]
 
@@ -678,6 +679,37 @@ def pack_rows(x: torch.Tensor) -> PackedRows:
     return out
 
 
+def decode_embed(
+    ids: torch.Tensor,        # [rows] int64 token ids
+    positions: torch.Tensor,  # [rows] int64
+    table: torch.Tensor,      # [vocab, hidden] fp16
+    inv_freq: torch.Tensor,   # [head_dim / 2] fp32 or fp16
+    scaling: float = 1.0,
+) -> Tuple[PackedRows, torch.Tensor, torch.Tensor]:
+    """A decode step's start in one launch: packed embedding rows, and rotary cos / sin rows.
+
+    embed_tokens and Qwen2RotaryEmbedding.forward with the same roundings; an id
+    outside the table gives a row of NaNs. cos and sin are [rows, head_dim] fp16.
+    """
+    assert ids.is_cuda and ids.dtype == torch.int64 and ids.dim() == 1 and ids.is_contiguous()
+    assert positions.dtype == torch.int64 and positions.shape == ids.shape
+    assert positions.is_contiguous() and table.dtype == torch.float16 and table.is_contiguous()
+    assert inv_freq.dtype in (torch.float32, torch.float16)
+    assert inv_freq.dim() == 1 and inv_freq.is_contiguous()
+    _native.same_device(ids, positions, table, inv_freq)
+    rows, (vocab, hidden), dim = ids.shape[0], table.shape, 2 * inv_freq.shape[0]
+    out = PackedRows(rows, hidden, 1, ids.device)
+    cos, sin = torch.empty(2, rows, dim, dtype=torch.float16, device=ids.device).unbind(0)
+    lib = _native.load()
+    with _on_device(ids.device):
+        status = lib.pa_decode_embed_f16(
+            ids.data_ptr(), positions.data_ptr(), table.data_ptr(), vocab, hidden,
+            inv_freq.data_ptr(), int(inv_freq.dtype == torch.float16), float(scaling), dim, out.data.data_ptr(), out.sums.data_ptr(),
+            cos.data_ptr(), sin.data_ptr(), rows, _native.stream_handle(ids.device))
+    _native.check(status, "pa_decode_embed_f16")
+    return out, cos, sin
+
+
 def decode_linear(
     x: Union[torch.Tensor, PackedRows],  # rows [rows, k]
     weight: torch.Tensor,                # pack_weight of [n, k]; with silu of [2 n, k] (gate, up)
@@ -863,6 +895,19 @@ def _stack_takes(self: nn.Module, input_ids, attention_mask, position_ids, past_
             and not any(_has_hooks(layer) for layer in self.layers))
 
 
+def _plain_embedding_and_rope(self: nn.Module) -> bool:
+    """Whether the base model's embedding and rotary modules are the plain ones decode_embed computes."""
+    emb, rope = self.embed_tokens, self.rotary_emb
+    return (type(emb) is nn.Embedding and emb.max_norm is None and not _has_hooks(emb)
+            and emb.weight.is_cuda and emb.weight.dtype == torch.float16
+            and emb.weight.is_contiguous() and emb.weight.data_ptr() % 16 == 0
+            and type(rope).__name__ == "Qwen2RotaryEmbedding" and not _has_hooks(rope)
+            and "forward" not in rope.__dict__ and "forward" not in emb.__dict__
+            and getattr(rope, "rope_type", None) == "default"
+            and rope.inv_freq.dtype in (torch.float32, torch.float16)
+            and rope.inv_freq.is_contiguous())
+
+
 def fused_decoder_stack_forward(
     self: nn.Module,
     input_ids: Optional[torch.Tensor] = None,
@@ -891,11 +936,18 @@ def fused_decoder_stack_forward(
     from transformers.modeling_outputs import BaseModelOutputWithPast
 
     ctx = self._paged_stack_context
-    x = self.embed_tokens(input_ids)
-    b, _, hidden = x.shape
-    cos, sin = self.rotary_emb(x, position_ids)
-    rows = pack_rows(x.view(b, hidden))
+    b = input_ids.shape[0]
     layers = self.layers[:self.config.num_hidden_layers]
+    if position_ids.shape == (b, 1) and position_ids.dtype == input_ids.dtype == torch.int64 and \
+            _plain_embedding_and_rope(self):
+        rows, cos, sin = decode_embed(input_ids.reshape(b).contiguous(),
+                                      position_ids.reshape(b).contiguous(),
+                                      self.embed_tokens.weight, self.rotary_emb.inv_freq,
+                                      self.rotary_emb.attention_scaling)
+    else:
+        x = self.embed_tokens(input_ids)
+        cos, sin = self.rotary_emb(x, position_ids)
+        rows = pack_rows(x.view(b, -1))
     for i, layer in enumerate(layers):
         attn, mlp = layer.self_attn, layer.mlp
         qkv_w, o_w, gu_w, down_w = layer._pa_packed
@@ -914,8 +966,7 @@ def fused_decoder_stack_forward(
         act = decode_linear(h, gu_w, norm=(norm2.weight, norm2.variance_epsilon), silu=True)
         last = i + 1 == len(layers)
         rows = decode_linear(act, down_w, residual=h, packed=not last, sums=not last)
-    x = rows if layers else x
-    return BaseModelOutputWithPast(last_hidden_state=self.norm(x.view(b, 1, hidden)))
+    return BaseModelOutputWithPast(last_hidden_state=self.norm(rows.view(b, 1, -1)))
 
 
 def _fused_rms_norm_forward(self: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:
@@ -951,6 +1002,7 @@ def patch_paged_attention(model: nn.Module, context: PagedAttentionContext,
             module.forward = fused_decoder_layer_forward.__get__(module, module.__class__)
             patched.append((module, orig_fwd, "layer"))
         elif decode and type(module).__name__ == "Qwen2Model" and \
+                len(module.layers) > 0 and \
                 all(hasattr(layer, "_pa_packed") for layer in module.layers):
             orig_fwd = module.forward
             module._orig_stack_forward = orig_fwd
@@ -1045,8 +1097,8 @@ def graph_batch_size(n: int) -> int:
 class _DecodeGraph:
     """One decode step captured as a HIP graph for a batch-size bucket and table width.
 
-    Static device buffers hold the step's inputs: token ids and lengths (one
-    pinned host-to-device copy per step, unpacked inside the graph) and the
+    Static device buffers hold the step's inputs: token ids, positions and
+    lengths (one pinned host-to-device copy per step) and the
     zero-padded block tables (copied only when a row changed: a sequence
     gained a block or the batch was reordered). Rows past the step's batch are
     padding with length 0. The graph replays the whole model forward -- each
@@ -1064,14 +1116,15 @@ class _DecodeGraph:
     def __init__(self, runner: "KernelPagedManualDecode", batch: int, width: int):
         dev = runner.device
         self.batch, self.width = batch, width
-        self.host_in = torch.zeros(2, batch, dtype=torch.long).pin_memory()  # ids, lengths
-        self.dev_in = torch.zeros(2, batch, dtype=torch.long, device=dev)
+        # Rows: token ids, positions, lengths (as int32 in the first half of their row).
+        self.host_in = torch.zeros(3, batch, dtype=torch.long).pin_memory()
+        self.dev_in = torch.zeros(3, batch, dtype=torch.long, device=dev)
         self.host_tables = torch.zeros(batch, width, dtype=torch.int32).pin_memory()
         self.tables = torch.zeros(batch, width, dtype=torch.int32, device=dev)
         self.mirror = np.full((batch, width), -1, dtype=np.int32)  # table contents on the device
-        self.ids = torch.zeros(batch, 1, dtype=torch.long, device=dev)
-        self.pos = torch.zeros(batch, 1, dtype=torch.long, device=dev)
-        self.lens = torch.ones(batch, dtype=torch.int32, device=dev)
+        self.ids = self.dev_in[0].view(-1, 1)
+        self.pos = self.dev_in[1].view(-1, 1)
+        self.lens = self.dev_in[2].view(torch.int32)[:batch]
         self.ctx = PagedAttentionContext.from_device(runner.pool, self.tables, self.lens,
                                                      runner.block_size)
         self.runner = runner
@@ -1080,9 +1133,6 @@ class _DecodeGraph:
         self.rows = 0
 
     def _body(self):
-        self.ids.copy_(self.dev_in[0].view(-1, 1))
-        self.lens.copy_(self.dev_in[1])
-        self.pos.copy_((self.dev_in[1] - 1).clamp_min(0).view(-1, 1))  # padding rows: position 0
         model = self.runner.model
         with patch_paged_attention(model, self.ctx, fuse_layers=self.runner.fuse_layers):
             out = model(input_ids=self.ids, position_ids=self.pos, use_cache=False)
@@ -1094,9 +1144,11 @@ class _DecodeGraph:
         assert n <= self.batch
         self.rows = n
         hin = self.host_in.numpy()
-        hin[:, n:] = 0
+        hin[:, n:] = 0  # padding rows: token 0 at position 0, length 0
         hin[0, :n] = tokens
         hin[1, :n] = lens
+        hin[2].view(np.int32)[:self.batch] = hin[1]
+        hin[1, :n] -= 1
         self.dev_in.copy_(self.host_in, non_blocking=True)
         # One vectorised scatter of all rows (a Python loop over 128 rows of
         # numpy slice assignments costs about 0.1 ms per step).
