@@ -123,3 +123,35 @@ def test_head_dim_32_single_head_tiles_span_blocks(cuda_device, hkv, g, bs, lens
                                            compute_dtype=torch.float32)
     err = (out.float().cpu() - want.float()).abs().max().item()
     assert err <= TOL, f"max abs err {err:.3e}"
+
+
+# Few pairs, each cut into many ranges (merges whose records are split over the threads): record
+# counts below, at and past a round of eight and past one round of every slice, one and several
+# slices (group size and head_dim), empty and one-token sequences among long ones, every block
+# specialisation, and more pairs than one launch's ranges.
+@pytest.mark.parametrize("d,hkv,g,bs,lens", [
+    (64, 2, 7, 16, [24001]),
+    (64, 2, 7, 32, [2049, 0, 12000, 1]),
+    (64, 1, 16, 8, [9000, 16 * 128 + 1]),
+    (64, 3, 1, 12, [5000, 700]),
+    (32, 2, 2, 16, [16384, 40]),
+    (32, 1, 16, 8, [7000]),
+    (128, 4, 7, 16, [3000, 17, 9001]),
+    (128, 2, 16, 32, [8001]),
+    (256, 2, 8, 16, [6000]),
+    (256, 1, 16, 8, [4000, 2500]),
+    (64, 16, 1, 16, [2100 + 31 * i for i in range(16)]),
+])
+def test_few_pairs_many_ranges(cuda_device, d, hkv, g, bs, lens):
+    c = dict(d=d, hkv=hkv, g=g, bs=bs, lens=lens, share=False, seed=d + hkv + g + bs)
+    q, k, v, bt, sl, tables, qc, kc, vc = build(c, cuda_device)
+    print(f"[few pairs] d={d} hkv={hkv} g={g} bs={bs} lens={lens}", flush=True)
+    out = paged_attention_decode_batched(q, k, v, bt, sl, d ** -0.5)
+    assert torch.equal(out, paged_attention_decode_batched(q, k, v, bt, sl, d ** -0.5))
+    live = [i for i, n in enumerate(lens) if n > 0]
+    assert all(torch.count_nonzero(out[i]).item() == 0 for i, n in enumerate(lens) if n == 0)
+    want = naive_reference_paged_attention(qc[live], kc, vc, [tables[i] for i in live],
+                                           [lens[i] for i in live], d ** -0.5,
+                                           compute_dtype=torch.float32)
+    err = (out[live].float().cpu() - want.float()).abs().max().item()
+    assert err <= TOL, f"max abs err {err:.3e}"

@@ -250,6 +250,22 @@ constexpr int kPairShortTiles = 64;
 // 17.7; 1 x 4096 16.0 against 17.8, 16.2 and 17.1; 1 x 8192 18.7 against 23.2,
 // 17.8 and 18.9; batches that fill the GPU unchanged.
 constexpr int kSkMinRange = 16;
+// Batches of at most this many pairs (at head_dim 128 and 256: kSkFewPairsWide)
+// take the kernel for few pairs, whose merges split a pair's rounds of records
+// over the threads, and at most kSkFewRanges ranges per pair: each more is
+// another record to merge. Measured on MI355X (launches in a captured graph,
+// two pools in turn, 14 q / 2 kv heads of 64 unless stated), the general kernel
+// against it, us: 1 x 2048 tokens 14.1 and 12.9, 8192 18.3 and 14.5, 24001 28.2
+// and 16.6, 32768 30.9 and 15.0; 2 x 12000 21.4 and 16.5; 4 x up to 16384 19.8
+// and 15.4; 8 x up to 3001 13.2 and 12.0; 60 x up to 4096 (120 pairs) 22.8 and
+// 22.5; head_dim 32, 16384 tokens 21.4 and 13.9; head_dim 256 31.3 and 29.3; 4
+// kv heads of 128, 24000 tokens 22.9 and 20.4, but 32 pairs of 6000 27.2 and
+// 27.6, 64 of up to 8192 32.6 and 33.0. Ranges per pair, 24, 32, 48, 64, 96:
+// 24001 tokens 18.1, 17.1, 16.6, 17.1, 18.1; 32768 17.9, 16.0, 15.0, 15.3, 16.4;
+// shorter contexts within 0.5 (their ranges are kSkMinRange positions).
+constexpr int kSkFewPairs = 256;
+constexpr int kSkFewPairsWide = 16;
+constexpr int kSkFewRanges = 48;
 
 // Compute units of the current device (cached per device; threads that race
 // on the first query store the same value).
@@ -300,6 +316,8 @@ static void streamk_plan(DecodeArgs& a, int num_seqs, int head_dim) {
   a.share = !a.pair_per_wg && streamk_may_share(num_seqs, head_dim, a.bs) &&
             streamk_can_share(a, head_dim);
   a.slot_recs = a.share && kPfxColBlocks > a.head_group ? kPfxColBlocks : a.head_group;
+  const int few = head_dim <= 64 ? kSkFewPairs : kSkFewPairsWide;
+  a.few_pairs = !a.share && a.head_group == 1 && pairs <= few ? pairs * kSkFewRanges : 0;
 }
 
 // Workspace bytes the planned launch touches: the pair counters, then two
@@ -643,7 +661,8 @@ int decode_batched(const void* q, const int64_t q_strides[3], const void* k_cach
       a.recs_bytes = rb < 0x7fffffffu ? (int)rb : 0x7fffffff;
       return finish_launch(launch_decode_write(a, *newrow, head_dim, (hipStream_t)stream));
     }
-    if (!plan_handover_supported(a, head_dim)) {
+    // (With few pairs the plan is short and every workgroup derives it.)
+    if (a.few_pairs || !plan_handover_supported(a, head_dim)) {
       const int rc = write_first();
       if (rc) return rc;
     } else {

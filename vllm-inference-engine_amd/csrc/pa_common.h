@@ -61,6 +61,10 @@ struct DecodeArgs {
   // lets the kernel find runs of neighbouring sequences whose leading table
   // entries are the same physical blocks and read those blocks once per run.
   int share;
+  // Nonzero: few pairs, each cut into many ranges (stream-K without sharing,
+  // one kv head per pair): the kernel whose merges split a pair's records over
+  // the threads, and the most ranges it may use.
+  int few_pairs;
   int max_members;  // sequences per sharing group (at most kPfxMaxMembers)
   int slot_recs;    // records per partial-record slot: max(head_group, kPfxColBlocks) when sharing
   // The stream-K plan (positions, then sharing information; layout of the

@@ -682,9 +682,29 @@ __device__ __forceinline__ void sk_plan(const DecodeArgs& a, const int NHG, int*
   }
 }
 
+// Records a thread combines by itself in a merge (one round of loads).
+constexpr int kMergeRound = 8;
+constexpr int kLongMerge = 1 << 30;  // marks a listed pair of more records (pair numbers stay below)
+
+__device__ inline void store_merged(f16* o, float den, f32x4 num) {
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  f16x4 ov;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) ov[c] = (f16)(num[c] * inv);
+  *reinterpret_cast<f16x4*>(o) = ov;
+}
+
 // PLAN_IN: the plan comes from a.plan_in (left by the K/V write launch just
 // before this one) instead of being derived by every workgroup.
-template <int D, int NT, int BS, int HG, int NW, bool PLAN_IN = false>
+// FEW: batches of few pairs (a.few_pairs), each cut into many ranges: no sharing
+// groups (fewer registers), no merge before the walk ends (a range never lists
+// more pairs than the list holds), and merges whose rounds are split over the
+// threads. One context of 24001 tokens is 48 records per kv head; with a thread
+// per output the last workgroup read them in rounds of eight, one memory round
+// trip after another, for about 10 of the launch's 28 us. In the general kernel
+// the same code cost the walk registers (99.5 against 97.9 us on the
+// long-context batch of 256).
+template <int D, int NT, int BS, int HG, int NW, bool PLAN_IN = false, bool FEW = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void decode_streamk_kernel(DecodeArgs a) {
   constexpr int NC = D / 32;
@@ -694,7 +714,7 @@ void decode_streamk_kernel(DecodeArgs a) {
   constexpr bool UNIFORM_TILE = BS > 0 && BS % 16 == 0;
   // Prefix items are built where a tile lies in one block and four column
   // blocks of accumulators fit the registers.
-  constexpr bool SHARE = UNIFORM_TILE && D <= 64;
+  constexpr bool SHARE = UNIFORM_TILE && D <= 64 && !FEW;
   constexpr int NCP = kPfxColBlocks;
   constexpr int NTP = 2;  // tiles per chunk of a prefix item (one kv head)
   constexpr int VST = NT * HG * 16 * LS;  // halves of one staging buffer (K or V) per wavefront
@@ -791,7 +811,8 @@ void decode_streamk_kernel(DecodeArgs a) {
   // Ranges: at least min_range tile positions each, at most one per
   // workgroup; workgroups beyond them get no range.
   const int T = uni(s_pos[B]);
-  const int Gw = (T + a.min_range - 1) / a.min_range;
+  int Gw = (T + a.min_range - 1) / a.min_range;
+  if constexpr (FEW) Gw = min(Gw, a.few_pairs);
   const int Ge = (int)(Gw < G ? Gw : G);  // 0 when every sequence is empty
 
   // The first Ge workgroups take part. Workgroup i is dispatched to XCD i % 8;
@@ -894,93 +915,128 @@ void decode_streamk_kernel(DecodeArgs a) {
     if (tid == 0) s_nmerge = 0;
     __syncthreads();
     if (tid < npend) {
-      int expect = 0;
+      int expect = 0, most = 0;
 #pragma unroll
       for (int hh = 0; hh < HG; ++hh) {
         Geo g;
         int wa_s, ns, wa_p, np;
         contributions(my_pair, hh, g, wa_s, ns, wa_p, np);
         expect += (hh == 0 ? ns : 0) + np;
+        most = max(most, ns + np);
       }
-      if (my_old == expect - 1) s_mlist[atomicAdd(&s_nmerge, 1)] = my_pair;
+      if (my_old == expect - 1)
+        s_mlist[atomicAdd(&s_nmerge, 1)] = my_pair | (FEW && most > kMergeRound ? kLongMerge : 0);
     }
     __syncthreads();
     const int nmg = s_nmerge;
     constexpr int DQ = D / 4;
     const int per = HG * a.g * DQ;
     const int mpb = 16 / a.g;
-    for (int it = tid; it < nmg * per; it += NTHR) {
-      // Item: four accumulators (dq) of query head qr of kv head h of one
-      // merged pair.
-      const int e = it / per;
-      int rem = it - e * per;
-      const int hh = rem / (a.g * DQ);
-      rem -= hh * a.g * DQ;
-      const int qr = rem / DQ;
-      const int dq = rem - qr * DQ;
-      const int p = s_mlist[e];
-      const int pb = p / NHG;
-      const int h = (p - pb * NHG) * HG + hh;
-      Geo g;
-      int wa_s, ns, wa_p, np;
-      contributions(p, hh, g, wa_s, ns, wa_p, np);
-      const int n = ns + np;
-      // Record k: a whole suffix or prefix item of a sharing member has its
-      // own record; cut items use range slots. A prefix item's record is one
-      // of its column blocks, whose 16 rows hold members cb * mpb .. cb * mpb +
-      // mpb - 1 times the query group: this member's rows start at rsh.
-      const int cbm = g.m / mpb;
-      const int rsh = (g.m - cbm * mpb) * a.g;
-      auto rec_of = [&](int k) -> int {
-        if (k < ns)
-          return (int)(ns == 1 ? QBASE + ((int64_t)pb * Hkv + h) * REC
-                               : slot_base(wa_s + k, k == 0) + (int64_t)hh * REC);
-        const int j = k - ns;
-        return (int)(np == 1 ? PBASE + ((int64_t)(pb - g.m + cbm) * Hkv + h) * REC
-                             : slot_base(wa_p + j, j == 0) + (int64_t)cbm * REC);
-      };
+    // Pairs of few records: a thread per item, all such pairs at once. A pair
+    // of more than kMergeRound: alone, with `slices` threads per item that take
+    // every slices-th round of eight records, and their sums combined through
+    // LDS in slice order -- one thread per item would make its rounds one
+    // memory round trip after another.
+    int slices = 1;
+    while (FEW && 2 * slices * per <= NTHR && slices < 8) slices *= 2;
+    for (int e0 = 0, cnt = 0; e0 < nmg; e0 += cnt) {
+      const bool alone = FEW && slices > 1 && (uni(s_mlist[e0]) & kLongMerge);
+      const int sl = alone ? slices : 1;
+      cnt = FEW ? 1 : nmg;
+      while (FEW && !alone && e0 + cnt < nmg && (slices == 1 || !(uni(s_mlist[e0 + cnt]) & kLongMerge))) ++cnt;
       float M = kNegInf, den = 0.f;
       f32x4 num = {0.f, 0.f, 0.f, 0.f};
-      for (int k0 = 0; k0 < n; k0 += 8) {
-        float mv[8], lv[8];
-        f32x4 av[8];
+      f16* o = nullptr;
+      for (int it = tid; it < cnt * per * sl; it += NTHR) {
+        // Item: four accumulators (dq) of query head qr of kv head h of one
+        // merged pair (and the slice).
+        const int e = it / per;
+        int rem = it - e * per;
+        const int hh = rem / (a.g * DQ);
+        rem -= hh * a.g * DQ;
+        const int qr = rem / DQ;
+        const int dq = rem - qr * DQ;
+        const int p = s_mlist[alone ? e0 : e0 + e] & (kLongMerge - 1);
+        const int pb = p / NHG;
+        const int h = (p - pb * NHG) * HG + hh;
+        Geo g;
+        int wa_s, ns, wa_p, np;
+        contributions(p, hh, g, wa_s, ns, wa_p, np);
+        const int n = ns + np;
+        // Record k: a whole suffix or prefix item of a sharing member has its
+        // own record; cut items use range slots. A prefix item's record is one
+        // of its column blocks, whose 16 rows hold members cb * mpb .. cb * mpb +
+        // mpb - 1 times the query group: this member's rows start at rsh.
+        const int cbm = g.m / mpb;
+        const int rsh = (g.m - cbm * mpb) * a.g;
+        auto rec_of = [&](int k) -> int {
+          if (k < ns)
+            return (int)(ns == 1 ? QBASE + ((int64_t)pb * Hkv + h) * REC
+                                 : slot_base(wa_s + k, k == 0) + (int64_t)hh * REC);
+          const int j = k - ns;
+          return (int)(np == 1 ? PBASE + ((int64_t)(pb - g.m + cbm) * Hkv + h) * REC
+                               : slot_base(wa_p + j, j == 0) + (int64_t)cbm * REC);
+        };
+        M = kNegInf;
+        den = 0.f;
+        num = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int k0 = alone ? 8 * e : 0; k0 < n; k0 += 8 * sl) {
+          float mv[8], lv[8];
+          f32x4 av[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          // Padding past the item's records reads at an offset past the record
-          // area: the buffer returns zeros and touches no memory.
-          const bool live = k0 + k < n;
-          const int kk = live ? k0 + k : 0;
-          const int base = rec_of(kk);
-          const int r = (kk < ns ? 0 : rsh) + qr;  // this query head's row of the record
-          constexpr int kOut = 0x7ffffff0;
-          mv[k] = load_coherent4(rec_rsrc, live ? 4 * (base + r) : kOut);
-          lv[k] = load_coherent4(rec_rsrc, live ? 4 * (base + 16 + r) : kOut);
-          av[k] = load_coherent16(rec_rsrc, live ? 4 * (base + 32 + r * D + dq * 4) : kOut);
-          if (!live) mv[k] = kNegInf;
+          for (int k = 0; k < 8; ++k) {
+            // Padding past the item's records reads at an offset past the record
+            // area: the buffer returns zeros and touches no memory.
+            const bool live = k0 + k < n;
+            const int kk = live ? k0 + k : 0;
+            const int base = rec_of(kk);
+            const int r = (kk < ns ? 0 : rsh) + qr;  // this query head's row of the record
+            constexpr int kOut = 0x7ffffff0;
+            mv[k] = load_coherent4(rec_rsrc, live ? 4 * (base + r) : kOut);
+            lv[k] = load_coherent4(rec_rsrc, live ? 4 * (base + 16 + r) : kOut);
+            av[k] = load_coherent16(rec_rsrc, live ? 4 * (base + 32 + r * D + dq * 4) : kOut);
+            if (!live) mv[k] = kNegInf;
+          }
+          float mb = M;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) mb = fmaxf(mb, mv[k]);
+          const float sc = M == kNegInf ? 0.f : fast_exp2(M - mb);
+          num *= sc;
+          den *= sc;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const float wk = mv[k] == kNegInf ? 0.f : fast_exp2(mv[k] - mb);
+            num += wk * av[k];
+            den += wk * lv[k];
+          }
+          M = mb;
         }
-        float mb = M;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) mb = fmaxf(mb, mv[k]);
-        const float sc = M == kNegInf ? 0.f : fast_exp2(M - mb);
-        num *= sc;
-        den *= sc;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float wk = mv[k] == kNegInf ? 0.f : fast_exp2(mv[k] - mb);
-          num += wk * av[k];
-          den += wk * lv[k];
-        }
-        M = mb;
+        o = a.out + (int64_t)pb * a.o_sb + (int64_t)(h * a.g + qr) * a.o_sh + dq * 4;
+        if (!alone) store_merged(o, den, num);
       }
-      const float inv = den > 0.f ? 1.f / den : 0.f;
-      f16x4 ov;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) ov[c] = (f16)(num[c] * inv);
-      *reinterpret_cast<f16x4*>(a.out + (int64_t)pb * a.o_sb +
-                                (int64_t)(h * a.g + qr) * a.o_sh + dq * 4) = ov;
+      if (alone) {
+        float* part = reinterpret_cast<float*>(smem);  // the staging buffers are free here
+        *reinterpret_cast<f32x4*>(&part[tid * 4]) = num;
+        part[NTHR * 4 + tid] = M;
+        part[NTHR * 5 + tid] = den;
+        __syncthreads();
+        if (tid < per) {
+          for (int k = 0; k < sl; ++k) M = fmaxf(M, part[NTHR * 4 + k * per + tid]);
+          den = 0.f;
+          num = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int k = 0; k < sl; ++k) {
+            const float m = part[NTHR * 4 + k * per + tid];
+            const float wk = m == kNegInf ? 0.f : fast_exp2(m - M);
+            num += wk * *reinterpret_cast<const f32x4*>(&part[(k * per + tid) * 4]);
+            den += wk * part[NTHR * 5 + k * per + tid];
+          }
+          store_merged(o, den, num);
+        }
+        __syncthreads();
+      }
     }
     for (int e = tid; e < nmg; e += NTHR)
-      __hip_atomic_store(a.cnt + s_mlist[e], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(a.cnt + (s_mlist[e] & (kLongMerge - 1)), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     npend = 0;
     ncounted = 0;
@@ -1056,7 +1112,9 @@ void decode_streamk_kernel(DecodeArgs a) {
   b = step == 0 ? b_first : (step == 1 ? b_pairs : b_cont);
   while (x < x_end) {
     // Room for this segment's arrivals in the pending list.
-    if (npend > NTHR - kPfxMaxMembers - HG) resolve();
+    if constexpr (!FEW) {
+      if (npend > NTHR - kPfxMaxMembers - HG) resolve();
+    }
     int kind, idx;
     int pstart, pend;
     Geo g;
@@ -1457,6 +1515,13 @@ constexpr int sk_chunk_tiles(int hg) {
 template <int D, int BS, int HG>
 hipError_t launch_sk(const DecodeArgs& a, hipStream_t s) {
   constexpr int NT = sk_chunk_tiles<D>(HG);
+  if constexpr (HG == 1) {
+    if (a.few_pairs && !a.pair_per_wg) {
+      decode_streamk_kernel<D, NT, BS, 1, kSkWaves, false, true>
+          <<<a.num_wg, 64 * kSkWaves, 0, s>>>(a);
+      return hipGetLastError();
+    }
+  }
   if (a.pair_per_wg)
     decode_pair_kernel<D, NT, BS, HG, kSkWaves, 0><<<a.num_wg, 64 * kSkWaves, 0, s>>>(a, RopeIn{});
   else
