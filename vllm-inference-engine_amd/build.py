@@ -3,7 +3,9 @@
 Compiles every HIP source under csrc/ with hipcc for gfx950 and links them into
 engine/kernels/libpa_gfx950.so, next to the ctypes loader that opens it, and the
 benchmark's read-bandwidth probes (probes/bw_probe.hip) into
-probes/libbw_probe_gfx950.so. Object files go to _build/ at the repository root. Run directly
+probes/libbw_probe_gfx950.so. The module that calls the library with torch
+tensors (host/pa_host.cpp, host code only) becomes engine/kernels/_pa_host.so,
+linked against the library. Object files go to _build/ at the repository root. Run directly
 (``python vllm-inference-engine_amd/build.py``) or through
 ``__graft_entry__.build()``.
 """
@@ -22,6 +24,8 @@ CSRC = PKG_DIR / "csrc"
 INCLUDE = REPO_ROOT / "include"
 BUILD_DIR = REPO_ROOT / "_build"
 LIB_PATH = PKG_DIR / "engine" / "kernels" / "libpa_gfx950.so"
+HOST_SRC = PKG_DIR / "host" / "pa_host.cpp"
+HOST_MODULE = LIB_PATH.with_name("_pa_host.so")
 PROBE_SRC = PKG_DIR / "probes" / "bw_probe.hip"
 PROBE_LIB = PKG_DIR / "probes" / "libbw_probe_gfx950.so"
 
@@ -78,6 +82,37 @@ def _compile_one(src: Path) -> Path:
     return obj
 
 
+def _compile_host() -> Path:
+    """Object file of the host module (g++: it holds no device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = BUILD_DIR / "pa_host.o"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           *(f"-isystem{p}" for p in include_paths()),
+           f"-isystem{sysconfig.get_paths()['include']}", "-c", str(HOST_SRC), "-o", str(obj)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC.name}:\n{proc.stdout}\n{proc.stderr}")
+    return obj
+
+
+def _link_host(obj: Path) -> None:
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = HOST_MODULE.with_suffix(".so.tmp")
+    cmd = ["g++", "-shared", str(obj), f"-L{LIB_PATH.parent}", f"-l:{LIB_PATH.name}",
+           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-Wl,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link of {HOST_MODULE.name} failed:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, HOST_MODULE)
+
+
 def _link(objs: list[Path], lib: Path) -> None:
     tmp = lib.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs),
@@ -94,10 +129,13 @@ def build(verbose: bool = False) -> Path:
     srcs = _sources()
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC}")
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 2)) as ex:
+        host = ex.submit(_compile_host)
         objs = list(ex.map(_compile_one, srcs + [PROBE_SRC]))
+        host_obj = host.result()
     _link(objs[:-1], LIB_PATH)
     _link(objs[-1:], PROBE_LIB)
+    _link_host(host_obj)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources and {PROBE_LIB}", file=sys.stderr)
     return LIB_PATH

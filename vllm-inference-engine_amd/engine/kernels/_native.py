@@ -10,6 +10,7 @@ There is no fallback: when the library is missing every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -116,6 +117,45 @@ def load() -> ctypes.CDLL:
                     f"{LIB_PATH} has ABI {ver}, the bindings expect {ABI_VERSION}; rebuild it")
             _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The module that calls the library with torch tensors in native code (host/pa_host.cpp)."""
+    global _host
+    if _host is None:
+        load()
+        path = LIB_PATH.with_name("_pa_host.so")
+        if not path.exists():
+            raise NativeLibraryError(
+                f"{path} is not built; run `python vllm-inference-engine_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("_pa_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
+
+
+def direct(name: str, first: torch.Tensor, *args):
+    """host().<name>(first, *args, workspace, stream) on the current stream of first's device.
+
+    None when the call is not a plain one (see host/pa_host.cpp), no
+    workspace exists for the stream yet, or first is not on a GPU: the caller
+    then checks and launches it itself.
+    """
+    index = first.get_device()
+    if index < 0 or _raw_stream is None:
+        return None
+    stream = _raw_stream(index)
+    buf = _workspaces.get((index, stream, WS_DECODE))
+    if buf is None:
+        return None
+    try:
+        return getattr(_host or host(), name)(first, *args, buf, stream)
+    except TypeError:  # something that is not a tensor: the caller's checks say what
+        return None
 
 
 def i64_array(values) -> ctypes.Array:

@@ -82,6 +82,9 @@ def paged_attention_decode_batched(
     inside the same launch. Asynchronous on the current stream, like the
     Triton launch it replaces; repeated calls return the same bits.
     """
+    out = _native.direct("decode", q, k_cache, v_cache, block_tables, seq_lens, float(scale))
+    if out is not None:
+        return out
     assert q.is_cuda and k_cache.is_cuda and v_cache.is_cuda
     assert block_tables.is_cuda and seq_lens.is_cuda
     _native.same_device(q, k_cache, v_cache, block_tables, seq_lens)

@@ -238,6 +238,10 @@ def paged_rope_decode_attention(
     group) pair run as one kernel launch; the others as those two launches.
     Returns [num_seqs, num_q_heads, head_dim]; asynchronous on the current stream.
     """
+    out = _native.direct("rope_decode", query, key, value, cos, sin, k_cache, v_cache, block_tables,
+                         seq_lens, float(scale))
+    if out is not None:
+        return out
     query = _as_rows(query)
     key = _as_rows(key)
     value = _as_rows(value)
@@ -317,6 +321,10 @@ def paged_decode_kv_write_attention(
     those two launches.
     Returns [num_seqs, num_q_heads, head_dim]; asynchronous on the current stream.
     """
+    out = _native.direct("kv_write_decode", query, key, value, k_cache, v_cache, block_tables,
+                         seq_lens, float(scale))
+    if out is not None:
+        return out
     query = _as_rows(query)
     key = _as_rows(key)
     value = _as_rows(value)
