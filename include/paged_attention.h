@@ -58,7 +58,7 @@ enum {
  * pa_decode_kv_write_batched_f16; 14: the decode workspace's head also holds the
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
  * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
- * 16: pa_decode_embed_f16). */
+ * 16: pa_decode_embed_f16; 17: pa_greedy_f16). */
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */
@@ -358,6 +358,10 @@ PA_API int pa_prefill_attention_f16(const void* q, const int64_t q_strides[3],
  * (torch.topk(row, 2).values, a repeated maximum counted twice), as fp32.
  * NaN logits are skipped (torch would rank them first); a one-entry row gives
  * top[2r+1] = -inf.
+ *
+ * pa_greedy_f16: the same selection at the end of a decode step: copy[r] =
+ * logits[r] (contiguous rows), out[r] = the arg-max's position and out[rows +
+ * r] = the maximum minus the second-largest value, as doubles.
  */
 PA_API int pa_rmsnorm_f16(const void* x, int64_t x_row_stride, const void* residual,
                           int64_t residual_row_stride, void* sum, int64_t sum_row_stride,
@@ -367,6 +371,8 @@ PA_API int pa_silu_mul_f16(const void* gate_up, int64_t gate_up_row_stride, void
                            int64_t out_row_stride, int rows, int inter, void* stream);
 PA_API int pa_top2_f16(const void* logits, int64_t row_stride, int rows, int vocab,
                        int64_t* index, float* top, void* stream);
+PA_API int pa_greedy_f16(const void* logits, int64_t row_stride, int rows, int vocab, void* copy,
+                         double* out, void* stream);
 
 /*
  * Projections of a decode step's transformer layer over packed operands. No

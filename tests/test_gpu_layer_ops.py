@@ -14,7 +14,12 @@ from __future__ import annotations
 import pytest
 import torch
 
-from engine.kernels.paged_attention_integration import greedy_top2, rms_norm, silu_mul
+from engine.kernels.paged_attention_integration import (
+    greedy_step,
+    greedy_top2,
+    rms_norm,
+    silu_mul,
+)
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +97,21 @@ def test_greedy_top2_matches_torch(cuda_device, rows, vocab):
     assert torch.equal(top, torch.topk(logits, 2, dim=-1).values.float())
     if vocab > 10:
         assert int(idx[0]) == 5 and float(top[0, 0] - top[0, 1]) == 0.0
+
+
+# Vocabulary sizes at the edges of the vector loop (eight values, 1024 threads, four loads each) and
+# off them, and rows of a wider buffer.
+@pytest.mark.parametrize("rows,vocab,pad", [
+    (1, 1, 0), (3, 8, 0), (2, 8191, 0), (5, 8192, 8), (4, 8200, 0), (3, 32768, 0), (2, 32776, 0),
+    (7, 151936, 64), (2, 1000, 3)])
+def test_greedy_step_is_top2_and_a_copy(cuda_device, rows, vocab, pad):
+    g = torch.Generator(device=cuda_device).manual_seed(vocab)
+    wide = torch.randn(rows, vocab + pad, generator=g, device=cuda_device).half()
+    logits = wide[:, :vocab]
+    logits[-1, vocab // 2] = logits[-1].max()  # a tie of the maximum
+    idx, top = greedy_top2(logits)
+    copy, both = greedy_step(logits)
+    assert torch.equal(copy, logits) and copy.is_contiguous()
+    assert torch.equal(both[0], idx.double())
+    assert torch.equal(both[1], top[:, 0].double() - top[:, 1].double())
+    assert torch.equal(idx, torch.argmax(logits, dim=-1))

@@ -427,7 +427,7 @@ using namespace pa;
 
 extern "C" {
 
-int pa_abi_version(void) { return 16; }
+int pa_abi_version(void) { return 17; }
 
 const char* pa_last_error(void) { return g_error.c_str(); }
 
@@ -1295,6 +1295,27 @@ int pa_top2_f16(const void* logits, int64_t row_stride, int rows, int vocab, int
   const bool vec = vocab % 8 == 0 && row_stride % 8 == 0 && aligned(logits, 16);
   return finish_launch(launch_top2((const f16*)logits, row_stride, rows, vocab, index, top, vec,
                                    (hipStream_t)stream));
+}
+
+int pa_greedy_f16(const void* logits, int64_t row_stride, int rows, int vocab, void* copy,
+                  double* out, void* stream) {
+  clear_error();
+  if (rows < 0 || vocab <= 0) {
+    set_error("rows must be >= 0 and vocab > 0");
+    return PA_ERR_ARG;
+  }
+  if (rows == 0) return PA_OK;
+  if (!logits || !copy || !out) {
+    set_error("null pointer argument");
+    return PA_ERR_ARG;
+  }
+  if (row_stride < vocab) {
+    set_error("row stride must be at least the vocabulary size");
+    return PA_ERR_ARG;
+  }
+  const bool vec = vocab % 8 == 0 && row_stride % 8 == 0 && aligned(logits, 16) && aligned(copy, 16);
+  return finish_launch(launch_greedy((const f16*)logits, row_stride, rows, vocab, (f16*)copy, out,
+                                     vec, (hipStream_t)stream));
 }
 
 int pa_pack_rows_f16(const void* x, int64_t x_row_stride, void* packed, float* row_sums, int rows,

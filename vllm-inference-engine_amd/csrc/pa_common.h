@@ -333,6 +333,8 @@ hipError_t launch_silu_mul(const f16* gu, int64_t gs, f16* out, int64_t os, int 
                            bool vec, hipStream_t s);
 hipError_t launch_top2(const f16* logits, int64_t ls, int rows, int V, int64_t* idx, float* top,
                        bool vec, hipStream_t s);
+hipError_t launch_greedy(const f16* logits, int64_t ls, int rows, int V, f16* copy, double* out,
+                         bool vec, hipStream_t s);
 
 // Length of sequence b clamped to [0, max_blocks * bs].
 __device__ inline int clamped_len(const DecodeArgs& a, int b) {

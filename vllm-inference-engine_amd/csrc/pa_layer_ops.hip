@@ -138,13 +138,22 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const f16* __restrict__ g
 // Per row of fp16 logits: the arg-max (first index of the maximum, as
 // torch.argmax returns it), the maximum and the second-largest value (the
 // top-2 of torch.topk, ties counted twice). One workgroup of 1024 threads per
-// row; with VEC, 16-byte loads of eight logits, two in flight per thread.
-template <bool VEC>
+// row; with VEC, 16-byte loads of eight logits, four in flight per thread.
+//
+// GREEDY: a decode step's end instead. The row is also copied to copy[r] (the
+// step's logits outlive the buffer they are computed in), and the result is
+// out[r] = the arg-max and out[rows + r] = maximum minus second, as doubles,
+// ready for the step's one transfer to the host: a copy of the logits, which
+// reads them again, and five small launches less per step.
+template <bool VEC, bool GREEDY>
 __global__ __launch_bounds__(1024) void top2_kernel(const f16* __restrict__ logits, int64_t ls,
                                                     int V, int64_t* __restrict__ idx,
-                                                    float* __restrict__ top) {
+                                                    float* __restrict__ top,
+                                                    f16* __restrict__ copy,
+                                                    double* __restrict__ out) {
   const int64_t r = blockIdx.x;
   const f16* row = logits + r * ls;
+  f16* crow = copy + r * V;
   const int tid = threadIdx.x;
   float m1 = -__builtin_huge_valf(), m2 = -__builtin_huge_valf();
   int i1 = 0x7fffffff;
@@ -159,19 +168,27 @@ __global__ __launch_bounds__(1024) void top2_kernel(const f16* __restrict__ logi
   };
   if constexpr (VEC) {
     const int nv = V / 8;
-    for (int j = tid; j < nv; j += 2048) {
-      const f16x8 a = *reinterpret_cast<const f16x8*>(row + 8 * j);
-      const bool two = j + 1024 < nv;
-      const f16x8 b = two ? *reinterpret_cast<const f16x8*>(row + 8 * (j + 1024)) : a;
+    constexpr int U = 4;
+    for (int j0 = tid; j0 < nv; j0 += U * 1024) {
+      f16x8 a[U];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) take((float)a[k], 8 * j + k);
-      if (two) {
+      for (int u = 0; u < U; ++u)
+        a[u] = *reinterpret_cast<const f16x8*>(row + 8 * min(j0 + u * 1024, nv - 1));
 #pragma unroll
-        for (int k = 0; k < 8; ++k) take((float)b[k], 8 * (j + 1024) + k);
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + u * 1024;
+        if (j < nv) {
+          if constexpr (GREEDY) *reinterpret_cast<f16x8*>(crow + 8 * j) = a[u];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) take((float)a[u][k], 8 * j + k);
+        }
       }
     }
   } else {
-    for (int i = tid; i < V; i += 1024) take((float)row[i], i);
+    for (int i = tid; i < V; i += 1024) {
+      if constexpr (GREEDY) crow[i] = row[i];
+      take((float)row[i], i);
+    }
   }
   // Combine (m1, i1, m2) across lanes: the larger maximum wins (lower index on
   // ties); the second value is the largest of the other three.
@@ -202,9 +219,14 @@ __global__ __launch_bounds__(1024) void top2_kernel(const f16* __restrict__ logi
     float a1 = s1[0], a2 = s2[0];
     int ai = si[0];
     for (int k = 1; k < 16; ++k) combine(a1, ai, a2, s1[k], si[k], s2[k]);
-    idx[r] = ai;
-    top[2 * r] = a1;
-    top[2 * r + 1] = a2;
+    if constexpr (GREEDY) {
+      out[r] = (double)ai;
+      out[gridDim.x + r] = (double)a1 - (double)a2;
+    } else {
+      idx[r] = ai;
+      top[2 * r] = a1;
+      top[2 * r + 1] = a2;
+    }
   }
 }
 
@@ -279,9 +301,18 @@ hipError_t launch_silu_mul(const f16* gu, int64_t gs, f16* out, int64_t os, int 
 hipError_t launch_top2(const f16* logits, int64_t ls, int rows, int V, int64_t* idx, float* top,
                        bool vec, hipStream_t s) {
   if (vec)
-    hipLaunchKernelGGL(top2_kernel<true>, dim3(rows), dim3(1024), 0, s, logits, ls, V, idx, top);
+    top2_kernel<true, false><<<rows, 1024, 0, s>>>(logits, ls, V, idx, top, nullptr, nullptr);
   else
-    hipLaunchKernelGGL(top2_kernel<false>, dim3(rows), dim3(1024), 0, s, logits, ls, V, idx, top);
+    top2_kernel<false, false><<<rows, 1024, 0, s>>>(logits, ls, V, idx, top, nullptr, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_greedy(const f16* logits, int64_t ls, int rows, int V, f16* copy, double* out,
+                         bool vec, hipStream_t s) {
+  if (vec)
+    top2_kernel<true, true><<<rows, 1024, 0, s>>>(logits, ls, V, nullptr, nullptr, copy, out);
+  else
+    top2_kernel<false, true><<<rows, 1024, 0, s>>>(logits, ls, V, nullptr, nullptr, copy, out);
   return hipGetLastError();
 }
 

@@ -18,7 +18,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_NAME = "libpa_gfx950.so"
 LIB_PATH = Path(__file__).with_name(LIB_NAME)
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 PA_OK = 0
 PA_ERR_ARG = 1
@@ -71,6 +71,7 @@ SIGNATURES: dict[str, tuple] = {
     "pa_rmsnorm_f16": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _f32,
                                _vp]),
     "pa_top2_f16": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp]),
+    "pa_greedy_f16": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp]),
     "pa_silu_mul_f16": (_i32, [_vp, _i64, _vp, _i64, _i32, _i32, _vp]),
     "pa_pack_rows_f16": (_i32, [_vp, _i64, _vp, _vp, _i32, _i32, _vp]),
     "pa_decode_embed_f16": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _i32, _f32, _i32, _vp, _vp, _vp,

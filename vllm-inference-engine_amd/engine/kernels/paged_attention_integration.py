@@ -61,6 +61,7 @@ __all__ = [
     "rms_norm",
     "silu_mul",
     "greedy_top2",
+    "greedy_step",
     "fused_decoder_stack_forward",
     "pack_weight",
     "pack_rows",
@@ -614,6 +615,26 @@ def greedy_top2(logits: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
                                  top.data_ptr(), _native.stream_handle(logits.device))
     _native.check(status, "pa_top2_f16")
     return idx, top
+
+
+def greedy_step(logits: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """A decode step's selection: (copy of the fp16 logits, [tokens, top-1 minus top-2] as float64).
+
+    greedy_top2 and the copy of the logits in one launch; float64 holds every
+    token id and every difference of two fp16 values exactly.
+    """
+    assert logits.is_cuda and logits.dtype == torch.float16 and logits.dim() == 2
+    assert logits.stride(-1) == 1
+    rows, vocab = logits.shape
+    copy = torch.empty(rows, vocab, dtype=torch.float16, device=logits.device)
+    out = torch.empty(2, rows, dtype=torch.float64, device=logits.device)
+    lib = _native.load()
+    with _on_device(logits.device):
+        status = lib.pa_greedy_f16(logits.data_ptr(), logits.stride(0), rows, vocab,
+                                   copy.data_ptr(), out.data_ptr(),
+                                   _native.stream_handle(logits.device))
+    _native.check(status, "pa_greedy_f16")
+    return copy, out
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
@@ -1468,7 +1489,7 @@ class KernelPagedManualDecode:
             width = max(64, -(-max(len(r) for r in rows) // 64) * 64)
             graph = self._decode_graph(n, width)
             graph.load(last_tokens, seq_lens, rows)
-            logits = graph.run().clone()  # the graph's output buffer is reused by the next step
+            logits = graph.run()
         else:
             input_ids = torch.tensor(last_tokens, dtype=torch.long, device=self.device).unsqueeze(1)
             position_ids = torch.tensor([[L - 1] for L in seq_lens], dtype=torch.long,
@@ -1479,11 +1500,13 @@ class KernelPagedManualDecode:
             logits = out.logits[:, -1, :]
         if logits.dtype == torch.float16 and logits.stride(-1) == 1:
             # torch.argmax and torch.topk(k=2) in one launch (their three
-            # multi-block reductions take about 0.17 ms at batch 128).
-            idx, top = greedy_top2(logits)
-            top2 = top.double()
-            both = torch.stack([idx.double(), top2[:, 0] - top2[:, 1]])
+            # multi-block reductions take about 0.17 ms at batch 128), which
+            # also copies the logits: the graph's output buffer is reused by
+            # the next step.
+            logits, both = greedy_step(logits)
         else:
+            if self.use_graphs:
+                logits = logits.clone()
             top2 = torch.topk(logits, k=2, dim=-1).values.double()
             both = torch.stack([torch.argmax(logits, dim=-1).double(), top2[:, 0] - top2[:, 1]])
         # float64 holds every token id exactly: tokens and margins in one transfer.
