@@ -58,7 +58,8 @@ enum {
  * pa_decode_kv_write_batched_f16; 14: the decode workspace's head also holds the
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
  * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
- * 16: pa_decode_embed_f16; 17: pa_greedy_f16). */
+ * 16: pa_decode_embed_f16; 17: pa_greedy_f16; 18:
+ * pa_decode_rope_prefetch_f16). */
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */
@@ -291,6 +292,25 @@ PA_API int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3],
                                       int num_q_heads, int num_kv_heads, int head_dim,
                                       int block_size, int num_blocks, int max_blocks_per_seq,
                                       float scale, void* workspace, size_t workspace_bytes,
+                                      void* stream);
+/* The same, and up to four ranges of device memory (16-byte aligned) that later
+ * launches on the stream will read -- the layer's next weights -- are read into the
+ * L2 caches meanwhile, as far as they fit, where the call runs as one launch. A
+ * hint: results do not depend on it. */
+PA_API int pa_decode_rope_prefetch_f16(const void* q, const int64_t q_strides[3], const void* key,
+                                      const int64_t key_strides[3], const void* value,
+                                      const int64_t value_strides[3], const void* cos,
+                                      const int64_t cos_strides[2], const void* sin,
+                                      const int64_t sin_strides[2], void* k_cache,
+                                      const int64_t k_strides[4], void* v_cache,
+                                      const int64_t v_strides[4], const int32_t* block_tables,
+                                      const int64_t bt_strides[2], const int32_t* seq_lens,
+                                      void* out, const int64_t out_strides[3], int num_seqs,
+                                      int num_q_heads, int num_kv_heads, int head_dim,
+                                      int block_size, int num_blocks, int max_blocks_per_seq,
+                                      float scale, void* workspace, size_t workspace_bytes,
+                                      const void* const* prefetch,
+                                      const int64_t* prefetch_bytes, int num_prefetch,
                                       void* stream);
 
 /*

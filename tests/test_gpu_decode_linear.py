@@ -168,3 +168,31 @@ def test_embed_matches_the_modules(cuda_device, rows, hidden, dim, freq):
         bad = torch.zeros(rows, dtype=torch.bool, device=cuda_device)
         bad[[1, rows - 1]] = True
         assert torch.isnan(out[bad]).all() and torch.equal(out[~bad], table[ids[~bad]])
+
+
+# Ranges of one load, ragged parts, an empty one, more than the L2 share; batches that leave CUs
+# free and that take the two-launch form (where nothing is fetched).
+@pytest.mark.parametrize("seqs,longest", [(1, 40), (9, 700), (128, 300), (1, 5000)])
+@pytest.mark.parametrize("sizes", [[16], [8, 1000, 0, 77777], [1 << 20, 40 << 20, 8]])
+def test_prefetch_changes_nothing(cuda_device, seqs, longest, sizes):
+    from engine.kernels.paged_attention_integration import paged_rope_decode_attention
+
+    g = torch.Generator(device=cuda_device).manual_seed(seqs)
+    width = -(-longest // 16)
+    blocks = seqs * width + 3
+    lens = torch.randint(1, longest + 1, (seqs,), generator=g, device=cuda_device).int()
+    lens[-1] = longest
+    tables = torch.randperm(blocks, generator=g, device=cuda_device)[:seqs * width]
+    tables = tables.view(seqs, width).int()
+    rows = [torch.randn(seqs, h, 64, generator=g, device=cuda_device).half() for h in (14, 2, 2)]
+    cos, sin = torch.randn(2, seqs, 64, generator=g, device=cuda_device).half()
+    pools = [torch.randn(blocks, 16, 2, 64, generator=g, device=cuda_device).half()
+             for _ in range(2)]
+    ranges = [torch.zeros(n // 2, dtype=torch.float16, device=cuda_device) for n in sizes]
+    results = []
+    for prefetch in ((), ranges):
+        own = [p.clone() for p in pools]
+        out = paged_rope_decode_attention(*rows, cos, sin, *own, tables, lens, 0.125,
+                                          prefetch=prefetch)
+        results.append((out, *own))
+    assert all(torch.equal(a, b) for a, b in zip(*results))

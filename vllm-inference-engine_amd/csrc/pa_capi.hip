@@ -427,7 +427,7 @@ using namespace pa;
 
 extern "C" {
 
-int pa_abi_version(void) { return 17; }
+int pa_abi_version(void) { return 18; }
 
 const char* pa_last_error(void) { return g_error.c_str(); }
 
@@ -996,7 +996,7 @@ size_t pa_decode_rope_batched_workspace_bytes(int num_seqs, int num_q_heads, int
   return ((ws + 255) & ~(size_t)255) + (size_t)num_seqs * num_q_heads * head_dim * 2;
 }
 
-int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const void* key,
+static int rope_batched(const void* q, const int64_t q_strides[3], const void* key,
                                const int64_t key_strides[3], const void* value,
                                const int64_t value_strides[3], const void* cos,
                                const int64_t cos_strides[2], const void* sin,
@@ -1007,7 +1007,8 @@ int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const 
                                const int64_t out_strides[3], int num_seqs, int num_q_heads,
                                int num_kv_heads, int head_dim, int block_size, int num_blocks,
                                int max_blocks_per_seq, float scale, void* workspace,
-                               size_t workspace_bytes, void* stream) {
+                               size_t workspace_bytes, const void* const* prefetch,
+                               const int64_t* prefetch_bytes, int num_prefetch, void* stream) {
   clear_error();
   if (num_seqs < 0) {
     set_error("num_seqs must be >= 0");
@@ -1020,6 +1021,16 @@ int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const 
     set_error("null pointer argument");
     return PA_ERR_ARG;
   }
+  if (num_prefetch < 0 || num_prefetch > kMaxPrefetch ||
+      (num_prefetch > 0 && (!prefetch || !prefetch_bytes))) {
+    set_error("at most %d ranges can be prefetched, %d given", kMaxPrefetch, num_prefetch);
+    return PA_ERR_ARG;
+  }
+  for (int i = 0; i < num_prefetch; ++i)
+    if (prefetch_bytes[i] < 0 || (prefetch_bytes[i] > 0 && (!prefetch[i] || !aligned(prefetch[i], 16)))) {
+      set_error("prefetch ranges need 16-byte aligned addresses and sizes >= 0");
+      return PA_ERR_ARG;
+    }
   int rc = check_common(q, k_cache, v_cache, out, k_strides, v_strides, num_q_heads, num_kv_heads,
                         head_dim, block_size, num_blocks);
   if (rc) return rc;
@@ -1100,6 +1111,17 @@ int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const 
   a.num_blocks = num_blocks;
   a.scale_log2 = scale * kLog2e;
   RopeIn r{};
+  // Within the L2s (4 MB per XCD, an eighth left for the attention itself), by
+  // workgroups on the CUs the attention leaves free, or a share of each if it
+  // fills them.
+  constexpr int64_t kPrefetchBytes = 28 << 20;
+  int64_t room = kPrefetchBytes;
+  for (int i = 0; i < num_prefetch && room > 0; ++i) {
+    r.prefetch[i] = prefetch[i];
+    r.prefetch_bytes[i] = prefetch_bytes[i] < room ? prefetch_bytes[i] : room;
+    room -= r.prefetch_bytes[i];
+  }
+  if (room < kPrefetchBytes) r.prefetch_wg = device_cus() / 8 * 8;
   r.key = (const f16*)key;
   r.ks_b = key_strides[0];
   r.ks_h = key_strides[1];
@@ -1111,6 +1133,45 @@ int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const 
   r.sin = (const f16*)sin;
   r.ss_b = sin_strides[0];
   return finish_launch(launch_decode_pair_rope(a, r, head_dim, (hipStream_t)stream));
+}
+
+int pa_decode_rope_batched_f16(const void* q, const int64_t q_strides[3], const void* key,
+                               const int64_t key_strides[3], const void* value,
+                               const int64_t value_strides[3], const void* cos,
+                               const int64_t cos_strides[2], const void* sin,
+                               const int64_t sin_strides[2], void* k_cache,
+                               const int64_t k_strides[4], void* v_cache,
+                               const int64_t v_strides[4], const int32_t* block_tables,
+                               const int64_t bt_strides[2], const int32_t* seq_lens, void* out,
+                               const int64_t out_strides[3], int num_seqs, int num_q_heads,
+                               int num_kv_heads, int head_dim, int block_size, int num_blocks,
+                               int max_blocks_per_seq, float scale, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+  return rope_batched(q, q_strides, key, key_strides, value, value_strides, cos, cos_strides, sin,
+                      sin_strides, k_cache, k_strides, v_cache, v_strides, block_tables, bt_strides,
+                      seq_lens, out, out_strides, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                      block_size, num_blocks, max_blocks_per_seq, scale, workspace, workspace_bytes,
+                      nullptr, nullptr, 0, stream);
+}
+
+int pa_decode_rope_prefetch_f16(const void* q, const int64_t q_strides[3], const void* key,
+                               const int64_t key_strides[3], const void* value,
+                               const int64_t value_strides[3], const void* cos,
+                               const int64_t cos_strides[2], const void* sin,
+                               const int64_t sin_strides[2], void* k_cache,
+                               const int64_t k_strides[4], void* v_cache,
+                               const int64_t v_strides[4], const int32_t* block_tables,
+                               const int64_t bt_strides[2], const int32_t* seq_lens, void* out,
+                               const int64_t out_strides[3], int num_seqs, int num_q_heads,
+                               int num_kv_heads, int head_dim, int block_size, int num_blocks,
+                               int max_blocks_per_seq, float scale, void* workspace,
+                               size_t workspace_bytes, const void* const* prefetch,
+                               const int64_t* prefetch_bytes, int num_prefetch, void* stream) {
+  return rope_batched(q, q_strides, key, key_strides, value, value_strides, cos, cos_strides, sin,
+                      sin_strides, k_cache, k_strides, v_cache, v_strides, block_tables, bt_strides,
+                      seq_lens, out, out_strides, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                      block_size, num_blocks, max_blocks_per_seq, scale, workspace, workspace_bytes,
+                      prefetch, prefetch_bytes, num_prefetch, stream);
 }
 
 size_t pa_prefill_attention_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads,

@@ -292,6 +292,7 @@ bool streamk_can_share(const DecodeArgs& a, int D);
 // rotary embedding): keys and values [num_seqs, kv heads, D] and the rotary
 // cos / sin rows [num_seqs, D], all with unit head_dim stride, 16-byte aligned
 // rows. Element strides.
+constexpr int kMaxPrefetch = 4;
 struct RopeIn {
   const f16* key;
   int64_t ks_b, ks_h;
@@ -301,6 +302,12 @@ struct RopeIn {
   int64_t cs_b;
   const f16* sin;
   int64_t ss_b;
+  // Memory the next launches read, fetched into the L2s meanwhile (one-launch
+  // rotary form only): each range in kXcds equal parts, part x by the
+  // prefetch_wg workgroups after the attention's that run on XCD x.
+  const void* prefetch[kMaxPrefetch];
+  int64_t prefetch_bytes[kMaxPrefetch];
+  int prefetch_wg;  // a multiple of the XCDs, 0: none
 };
 // Whether the fused decode-layer kernel serves the launch planned in `a`
 // (one workgroup per pair, head_dim 64 or 128, block 16 or 32), and its

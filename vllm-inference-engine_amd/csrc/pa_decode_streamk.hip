@@ -1300,6 +1300,38 @@ struct PairSeg {
   }
 };
 
+// Fetches this workgroup's share of the ranges a.prefetch names into its XCD's
+// L2: rank `rank` of `ranks` workgroups on XCD `xcd`.
+//
+// A small batch's attention leaves most CUs and the memory idle for its 9 us,
+// and the projections after it are bound by their weight streams: read from L2
+// they take (8 rows, hidden 896) 4.3 instead of 6.6 us (gate/up), 4.4 instead of
+// 5.5 (down), 2.9 instead of 3.2 (o); at 128 rows 8.1 instead of 10.8, 5.9
+// instead of 7.0, 4.1 instead of 4.5. Whole decode steps: 8 streams 919 -> 845
+// us, 128 streams (whose attention fills the CUs) 1363 -> 1326. The parts match
+// the consumers' workgroup order (xcd_order over column tiles); L2 contents
+// stay across launches.
+__device__ __forceinline__ void prefetch_ranges(const RopeIn& r, int xcd, int rank, int ranks,
+                                                int nthr) {
+  constexpr int U = 8;  // loads in flight
+#pragma unroll
+  for (int i = 0; i < kMaxPrefetch; ++i) {
+    const int64_t part = (r.prefetch_bytes[i] / kXcds + 127) & ~(int64_t)127;
+    const int64_t lo = min(xcd * part, r.prefetch_bytes[i]);
+    const int n = (int)min(part, r.prefetch_bytes[i] - lo);
+    if (n <= 0) continue;
+    const auto rs = tile_rsrc((const char*)r.prefetch[i] + lo, n);  // loads past it touch no memory
+    const int step = ranks * nthr * 16;
+    for (int o = (rank * nthr + (int)threadIdx.x) * 16; o < n; o += U * step) {
+      u32x4 v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + u * step, 0, 0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" ::"v"(v[u]));  // a use, or the loads would go
+    }
+  }
+}
+
 // Batched decode with one workgroup per (sequence, kv-head group) pair, for
 // batches whose pairs fill the GPU and are short (the schedule the C API
 // picks for them): no plan and no partial records. Workgroup w takes pair w
@@ -1337,7 +1369,12 @@ void decode_pair_kernel(DecodeArgs a, RopeIn r) {
   const int grp = lane >> 4;
   const int NHG = a.hkv / HG;
   const int P = a.num_seqs * NHG;
-  if ((int)blockIdx.x >= P) return;
+  if ((int)blockIdx.x >= P) {
+    if constexpr (ROPE)
+      prefetch_ranges(r, blockIdx.x % kXcds, (blockIdx.x - P) / kXcds, r.prefetch_wg / kXcds,
+                      64 * NW);
+    return;
+  }
   const int wg = xcd_order(blockIdx.x, P);
   const int b = wg / NHG;
   const int h0 = (wg - b * NHG) * HG;
@@ -1539,7 +1576,8 @@ hipError_t launch_sk_plan_in(const DecodeArgs& a, hipStream_t s) {
 template <int D, int BS, int HG>
 hipError_t launch_pair_rope(const DecodeArgs& a, const RopeIn& r, hipStream_t s) {
   constexpr int NT = sk_chunk_tiles<D>(HG);
-  decode_pair_kernel<D, NT, BS, HG, kSkWaves, 2><<<a.num_wg, 64 * kSkWaves, 0, s>>>(a, r);
+  decode_pair_kernel<D, NT, BS, HG, kSkWaves, 2>
+      <<<a.num_wg + r.prefetch_wg, 64 * kSkWaves, 0, s>>>(a, r);
   return hipGetLastError();
 }
 

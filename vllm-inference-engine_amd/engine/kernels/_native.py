@@ -18,7 +18,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_NAME = "libpa_gfx950.so"
 LIB_PATH = Path(__file__).with_name(LIB_NAME)
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 PA_OK = 0
 PA_ERR_ARG = 1
@@ -82,6 +82,10 @@ SIGNATURES: dict[str, tuple] = {
         _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
         _vp, _i64p, _vp, _vp, _i64p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp, _sz,
         _vp]),
+    "pa_decode_rope_prefetch_f16": (_i32, [
+        _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
+        _vp, _i64p, _vp, _vp, _i64p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp, _sz,
+        ctypes.POINTER(ctypes.c_void_p), _i64p, _i32, _vp]),
     "pa_decode_rope_batched_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "pa_decode_batched_noalloc_f16": (_i32, [
         _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _vp, _i64p,

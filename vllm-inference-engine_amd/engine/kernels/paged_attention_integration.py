@@ -24,12 +24,13 @@ layer (reference pad + index_copy_, :278-326).
 """
 from __future__ import annotations
 
+import ctypes
 import itertools
 import logging
 import math
 from collections import OrderedDict
 from contextlib import contextmanager
-from typing import Any, Callable, Dict, List, Optional, Tuple, Union
+from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
@@ -228,6 +229,7 @@ def paged_rope_decode_attention(
     block_tables: torch.Tensor,  # [num_seqs, max_blocks_per_seq] int32
     seq_lens: torch.Tensor,      # [num_seqs] int32, lengths including the new token
     scale: float,
+    prefetch: Sequence[torch.Tensor] = (),  # up to 4 contiguous tensors the next launches read
 ) -> torch.Tensor:
     """One decode step's attention block of a layer, in one call.
 
@@ -236,13 +238,16 @@ def paged_rope_decode_attention(
     on the rotated queries -- the reference's apply_rotary_pos_emb
     (integration.py:108-109), K/V write loop (:148-161) and batched attention
     call (:164-171). Batches that take one workgroup per (sequence, kv-head
-    group) pair run as one kernel launch; the others as those two launches.
+    group) pair run as one kernel launch; the others as those two launches. The
+    tensors of `prefetch` are read into the L2 caches meanwhile, as far as they
+    fit and where the call is one launch (a hint: results do not depend on it).
     Returns [num_seqs, num_q_heads, head_dim]; asynchronous on the current stream.
     """
-    out = _native.direct("rope_decode", query, key, value, cos, sin, k_cache, v_cache, block_tables,
-                         seq_lens, float(scale))
-    if out is not None:
-        return out
+    if not prefetch:
+        out = _native.direct("rope_decode", query, key, value, cos, sin, k_cache, v_cache,
+                             block_tables, seq_lens, float(scale))
+        if out is not None:
+            return out
     query = _as_rows(query)
     key = _as_rows(key)
     value = _as_rows(value)
@@ -252,7 +257,9 @@ def paged_rope_decode_attention(
         assert t.is_cuda and t.dtype == torch.float16
     assert block_tables.dtype == torch.int32 and block_tables.is_cuda and block_tables.dim() == 2
     assert seq_lens.is_cuda and seq_lens.dtype == torch.int32
-    _native.same_device(query, key, value, cos, sin, k_cache, v_cache, block_tables, seq_lens)
+    _native.same_device(query, key, value, cos, sin, k_cache, v_cache, block_tables, seq_lens,
+                        *prefetch)
+    assert len(prefetch) <= 4 and all(t.is_contiguous() for t in prefetch)
     assert k_cache.shape == v_cache.shape, "k_cache and v_cache must have the same shape"
     num_blocks, block_size, num_kv_heads, head_dim = k_cache.shape
     num_seqs, num_q_heads = query.shape[0], query.shape[1]
@@ -276,7 +283,9 @@ def paged_rope_decode_attention(
         if ws_bytes is None:
             ws_bytes = _rope_ws_sizes[ws_key] = lib.pa_decode_rope_batched_workspace_bytes(
                 *ws_key[1:])
-        status = lib.pa_decode_rope_batched_f16(
+        ptrs = (ctypes.c_void_p * max(1, len(prefetch)))(*(t.data_ptr() for t in prefetch))
+        sizes = _native.i64_array([t.numel() * t.element_size() for t in prefetch] or [0])
+        status = lib.pa_decode_rope_prefetch_f16(
             query.data_ptr(), _native.strides_of(query),
             key.data_ptr(), _native.strides_of(key),
             value.data_ptr(), _native.strides_of(value),
@@ -288,8 +297,8 @@ def paged_rope_decode_attention(
             seq_lens.data_ptr(), out.data_ptr(), _native.strides_of(out),
             num_seqs, num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, max_blocks,
             float(scale), _native.workspace(ws_bytes, dev, stream, _native.WS_DECODE), ws_bytes,
-            stream)
-    _native.check(status, "pa_decode_rope_batched_f16")
+            ptrs, sizes, len(prefetch), stream)
+    _native.check(status, "pa_decode_rope_prefetch_f16")
     return out
 
 
@@ -990,7 +999,8 @@ def fused_decoder_stack_forward(
         o = paged_rope_decode_attention(
             qkv[:, :nq * hd].view(b, nq, hd), qkv[:, nq * hd:(nq + nkv) * hd].view(b, nkv, hd),
             qkv[:, (nq + nkv) * hd:].view(b, nkv, hd), cos, sin, ctx.pool.k_cache[attn.layer_idx],
-            ctx.pool.v_cache[attn.layer_idx], ctx.padded_block_tables, ctx.seq_lens_tensor, scale)
+            ctx.pool.v_cache[attn.layer_idx], ctx.padded_block_tables, ctx.seq_lens_tensor, scale,
+            prefetch=(o_w, *gu_w.chunk(2), down_w))
         h = decode_linear(o.view(b, nq * hd), o_w, bias=attn.o_proj.bias, residual=rows, sums=True)
         act = decode_linear(h, gu_w, norm=(norm2.weight, norm2.variance_epsilon), silu=True)
         last = i + 1 == len(layers)
