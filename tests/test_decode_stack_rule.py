@@ -1,0 +1,62 @@
+"""Which calls of the base model the fused decode stack takes (no GPU needed)."""
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from engine.kernels.paged_attention_integration import DECODE_LINEAR_MAX_ROWS, _stack_takes
+
+
+@pytest.fixture(scope="module")
+def model():
+    from transformers import Qwen2Config
+    from transformers.models.qwen2.modeling_qwen2 import Qwen2Model
+
+    m = Qwen2Model(Qwen2Config(vocab_size=32, hidden_size=32, intermediate_size=32,
+                               num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=1))
+    m._paged_stack_context = SimpleNamespace(is_decode=True, is_batched=True)
+    return m
+
+
+def _takes(model, rows=3, width=1, mask=None, positions=True, cache=None, embeds=None,
+           use_cache=False, **kwargs):
+    ids = torch.zeros(rows, width, dtype=torch.long)
+    return _stack_takes(model, ids, mask, torch.zeros(rows, 1) if positions else None, cache,
+                        embeds, use_cache, kwargs)
+
+
+def test_plain_decode_steps_are_taken(model):
+    assert _takes(model) and _takes(model, rows=DECODE_LINEAR_MAX_ROWS)
+    assert _takes(model, output_hidden_states=False, cache_position=None)
+
+
+@pytest.mark.parametrize("call", [
+    dict(rows=DECODE_LINEAR_MAX_ROWS + 1), dict(rows=0), dict(width=2), dict(mask=torch.ones(3, 1)),
+    dict(positions=False), dict(cache=object()), dict(embeds=torch.zeros(3, 1, 32)),
+    dict(use_cache=True), dict(output_hidden_states=True), dict(output_attentions=True),
+    dict(cache_position=torch.arange(3)), dict(cache_position=torch.zeros(1)),
+])
+def test_calls_that_ask_for_more_take_the_layers(model, call):
+    assert not _takes(model, **call)
+
+
+def test_hooks_and_contexts_take_the_layers(model):
+    for register in (model.layers[1].register_forward_hook,
+                     model.layers[0].register_forward_pre_hook):
+        handle = register(lambda *a: None)
+        assert not _takes(model)
+        handle.remove()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not _takes(model)
+    handle.remove()
+    for context in (None, SimpleNamespace(is_decode=False, is_batched=True),
+                    SimpleNamespace(is_decode=True, is_batched=False)):
+        own, model._paged_stack_context = model._paged_stack_context, context
+        assert not _takes(model)
+        model._paged_stack_context = own
+    model.config.output_hidden_states = True
+    assert not _takes(model)
+    model.config.output_hidden_states = False
+    assert _takes(model)

@@ -926,7 +926,8 @@ def _stack_takes(self: nn.Module, input_ids, attention_mask, position_ids, past_
             and input_ids is not None and input_ids.dim() == 2 and input_ids.shape[1] == 1
             and 0 < input_ids.shape[0] <= DECODE_LINEAR_MAX_ROWS
             and attention_mask is None and position_ids is not None and past_key_values is None
-            and inputs_embeds is None and not use_cache and not any(kwargs.values())
+            and inputs_embeds is None and not use_cache
+            and all(v is None or v is False for v in kwargs.values())
             and not getattr(self.config, "output_hidden_states", False)
             and not getattr(self.config, "output_attentions", False)
             and not _module._global_forward_hooks and not _module._global_forward_pre_hooks
