@@ -1112,8 +1112,12 @@ static int rope_batched(const void* q, const int64_t q_strides[3], const void* k
   a.scale_log2 = scale * kLog2e;
   RopeIn r{};
   // Within the L2s (4 MB per XCD, an eighth left for the attention itself), by
-  // workgroups on the CUs the attention leaves free, or a share of each if it
-  // fills them.
+  // three eighths of the CUs' number of workgroups where the attention leaves
+  // half of the CUs free, else five eighths. Measured on MI355X, GPU time of a
+  // whole decode step (64, 96, 128, 160, 256 workgroups): 8 streams 777, 731,
+  // 737, 748, 755 us, 128 streams 1141, 1112, 1085, 1068, 1071; with 20 and 10 MB
+  // instead of 28 (128 workgroups) 793 and 818, 1119 and 1101. The next layer's
+  // q/k/v weights as well: 733 and 1091 (128).
   constexpr int64_t kPrefetchBytes = 28 << 20;
   int64_t room = kPrefetchBytes;
   for (int i = 0; i < num_prefetch && room > 0; ++i) {
@@ -1121,7 +1125,10 @@ static int rope_batched(const void* q, const int64_t q_strides[3], const void* k
     r.prefetch_bytes[i] = prefetch_bytes[i] < room ? prefetch_bytes[i] : room;
     room -= r.prefetch_bytes[i];
   }
-  if (room < kPrefetchBytes) r.prefetch_wg = device_cus() / 8 * 8;
+  if (room < kPrefetchBytes) {
+    const int cus = device_cus();
+    r.prefetch_wg = (2 * a.num_wg <= cus ? cus * 3 / 8 : cus * 5 / 8) / kXcdCount * kXcdCount;
+  }
   r.key = (const f16*)key;
   r.ks_b = key_strides[0];
   r.ks_h = key_strides[1];

@@ -1307,8 +1307,8 @@ struct PairSeg {
 // and the projections after it are bound by their weight streams: read from L2
 // they take (8 rows, hidden 896) 4.3 instead of 6.6 us (gate/up), 4.4 instead of
 // 5.5 (down), 2.9 instead of 3.2 (o); at 128 rows 8.1 instead of 10.8, 5.9
-// instead of 7.0, 4.1 instead of 4.5. Whole decode steps: 8 streams 919 -> 845
-// us, 128 streams (whose attention fills the CUs) 1363 -> 1326. The parts match
+// instead of 7.0, 4.1 instead of 4.5. Whole decode steps: 8 streams 919 -> 820
+// us, 128 streams (whose attention fills the CUs) 1363 -> 1324. The parts match
 // the consumers' workgroup order (xcd_order over column tiles); L2 contents
 // stay across launches.
 __device__ __forceinline__ void prefetch_ranges(const RopeIn& r, int xcd, int rank, int ranks,

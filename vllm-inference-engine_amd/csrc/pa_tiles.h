@@ -7,7 +7,7 @@
 namespace pa {
 namespace tiles {
 
-constexpr int kXcds = 8;  // accelerator complex dies of an MI355X, each with its own L2
+constexpr int kXcds = kXcdCount;
 
 // Position of workgroup i among n in an order in which each XCD (workgroup i
 // runs on XCD i % 8) owns a contiguous run of positions.
