@@ -36,7 +36,7 @@ def test_plain_decode_steps_are_taken(model):
     dict(rows=DECODE_LINEAR_MAX_ROWS + 1), dict(rows=0), dict(width=2), dict(mask=torch.ones(3, 1)),
     dict(positions=False), dict(cache=object()), dict(embeds=torch.zeros(3, 1, 32)),
     dict(use_cache=True), dict(output_hidden_states=True), dict(output_attentions=True),
-    dict(cache_position=torch.arange(3)), dict(cache_position=torch.zeros(1)),
+    dict(return_dict=False), dict(use_cache=None), dict(cache_position=torch.arange(3)), dict(cache_position=torch.zeros(1)),
 ])
 def test_calls_that_ask_for_more_take_the_layers(model, call):
     assert not _takes(model, **call)
@@ -60,3 +60,25 @@ def test_hooks_and_contexts_take_the_layers(model):
     assert not _takes(model)
     model.config.output_hidden_states = False
     assert _takes(model)
+
+
+@pytest.mark.parametrize("config", [{}, {"use_cache": False}, {"return_dict": False}])
+@pytest.mark.parametrize("call", [
+    {}, {"use_cache": None}, {"use_cache": False}, {"use_cache": False, "return_dict": None},
+    {"use_cache": False, "return_dict": True}, {"use_cache": False, "return_dict": False}])
+def test_calls_taken_return_hidden_states_alone(config, call):
+    """What the replaced forward returns, wherever the stack takes its call: a model output that
+    holds the last hidden states and nothing else."""
+    from transformers import Qwen2Config
+    from transformers.modeling_outputs import BaseModelOutputWithPast
+    from transformers.models.qwen2.modeling_qwen2 import Qwen2Model
+
+    m = Qwen2Model(Qwen2Config(vocab_size=32, hidden_size=32, intermediate_size=32,
+                               num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
+                               **config))
+    m._paged_stack_context = SimpleNamespace(is_decode=True, is_batched=True)
+    ids, pos = torch.zeros(3, 1, dtype=torch.long), torch.zeros(3, 1, dtype=torch.long)
+    out = m(input_ids=ids, position_ids=pos, **call)
+    alone = isinstance(out, BaseModelOutputWithPast) and list(out.keys()) == ["last_hidden_state"]
+    kwargs = {k: v for k, v in call.items() if k != "use_cache"}
+    assert _stack_takes(m, ids, None, pos, None, None, call.get("use_cache"), kwargs) == alone

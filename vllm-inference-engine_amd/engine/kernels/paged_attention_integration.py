@@ -922,12 +922,16 @@ def _stack_takes(self: nn.Module, input_ids, attention_mask, position_ids, past_
     ctx = self._paged_stack_context
     from torch.nn.modules import module as _module
 
+    # Left open by the caller, both are the configuration's to say, as in the forward replaced.
+    if use_cache is None:
+        use_cache = getattr(self.config, "use_cache", False)
+    return_dict = kwargs.get("return_dict", getattr(self.config, "return_dict", True))
     return (ctx is not None and ctx.is_decode and ctx.is_batched
             and input_ids is not None and input_ids.dim() == 2 and input_ids.shape[1] == 1
             and 0 < input_ids.shape[0] <= DECODE_LINEAR_MAX_ROWS
             and attention_mask is None and position_ids is not None and past_key_values is None
-            and inputs_embeds is None and not use_cache
-            and all(v is None or v is False for v in kwargs.values())
+            and inputs_embeds is None and not use_cache and return_dict is not False
+            and all(v is None or v is False or k == "return_dict" for k, v in kwargs.items())
             and not getattr(self.config, "output_hidden_states", False)
             and not getattr(self.config, "output_attentions", False)
             and not _module._global_forward_hooks and not _module._global_forward_pre_hooks
@@ -963,7 +967,7 @@ def fused_decoder_stack_forward(
     the residual stream kept packed between the launches: input norm + q/k/v;
     RoPE, K/V write and paged attention; o + residual; post-attention norm +
     gate/up + SwiGLU; down + residual. Calls that ask for more than a decode
-    step's hidden states (masks, caches, hidden-state outputs), layers with
+    step's hidden states (masks, caches, hidden-state outputs, tuples), layers with
     forward hooks and more than DECODE_LINEAR_MAX_ROWS rows take the layers one
     by one as before.
     """
