@@ -6,7 +6,12 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-from engine.kernels.paged_attention_integration import DECODE_LINEAR_MAX_ROWS, _stack_takes
+from engine.kernels.paged_attention_integration import (
+    DECODE_LINEAR_MAX_ROWS,
+    PagedAttentionContext,
+    _ids_checked,
+    _stack_takes,
+)
 
 
 @pytest.fixture(scope="module")
@@ -82,3 +87,13 @@ def test_calls_taken_return_hidden_states_alone(config, call):
     alone = isinstance(out, BaseModelOutputWithPast) and list(out.keys()) == ["last_hidden_state"]
     kwargs = {k: v for k, v in call.items() if k != "use_cache"}
     assert _stack_takes(m, ids, None, pos, None, None, call.get("use_cache"), kwargs) == alone
+
+
+def test_only_ids_checked_against_the_table_skip_the_embedding_module():
+    emb = torch.nn.Embedding(8, 4)
+    pool = SimpleNamespace(device=torch.device("cpu"))
+    ctx = PagedAttentionContext.from_device(pool, None, None)
+    assert not _ids_checked(ctx, emb) and not _ids_checked(SimpleNamespace(), emb)
+    for checked, taken in ((8, True), (5, True), (9, False)):
+        ctx.checked_vocab = checked
+        assert _ids_checked(ctx, emb) == taken

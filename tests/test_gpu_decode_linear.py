@@ -142,6 +142,41 @@ def test_stack_and_layer_paths_agree(cuda_device):
     assert diff <= 20 * 2.0 ** -11
 
 
+@pytest.mark.parametrize("use_graphs", [False, True])
+def test_ids_nobody_checked_go_through_the_embedding_module(cuda_device, monkeypatch, use_graphs):
+    """decode_step refuses ids outside the table and embeds the others in the step's first launch; a
+    model call with ids of its own asks the module, which refuses them as it always does."""
+    from engine import workloads
+    from engine.kernels import paged_attention_integration as integration
+    from engine.memory.block_allocator import BlockTable
+
+    launches = []
+    embed = integration.decode_embed
+    monkeypatch.setattr(integration, "decode_embed", lambda *a: launches.append(1) or embed(*a))
+    config = dict(vocab_size=512, hidden_size=128, intermediate_size=256, num_hidden_layers=1,
+                  num_attention_heads=4, num_key_value_heads=2, max_position_embeddings=4096,
+                  rope_theta=1e6, tie_word_embeddings=False)
+    with torch.inference_mode():
+        model = workloads.decode_model(cuda_device, 12, config)
+        runner = integration.KernelPagedManualDecode(model, num_blocks=8, device=str(cuda_device),
+                                                     use_graphs=use_graphs)
+        seq = {"seq_id": 0, "block_table": BlockTable(0, 16, [3], 5), "last_token_id": 511}
+        runner.pool.k_cache[0].zero_(), runner.pool.v_cache[0].zero_()
+        runner.decode_step([seq])
+        assert launches
+        with pytest.raises(IndexError):
+            runner.decode_step([dict(seq, last_token_id=512)])
+        launches.clear()
+        ctx = integration.PagedAttentionContext(runner.pool, [seq["block_table"]], [6])
+        with integration.patch_paged_attention(model, ctx):
+            out = model(input_ids=torch.full((1, 1), 511, device=cuda_device),
+                        position_ids=torch.full((1, 1), 5, device=cuda_device), use_cache=False)
+        assert not launches
+    # The same embedding row; rotary rows an fp16 rounding apart at most (2^-11 of a row's key).
+    diff = (out.logits[0, -1].float() - seq["last_logits"].float()).norm()
+    assert diff <= 2.0 ** -10 * seq["last_logits"].float().norm()
+
+
 @pytest.mark.parametrize("rows,hidden,dim,freq", [
     (1, 32, 64, torch.float32), (17, 896, 64, torch.float16), (130, 2336, 128, torch.float32)])
 def test_embed_matches_the_modules(cuda_device, rows, hidden, dim, freq):

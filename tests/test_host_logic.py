@@ -96,6 +96,26 @@ def test_runner_refuses_writes_without_a_block_or_into_shared_blocks():
         runner.prefill(SimpleNamespace(prompt_token_ids=None, prompt=None, block_table=shared))
 
 
+def test_runner_refuses_token_ids_outside_the_vocabulary():
+    """As an embedding lookup on the CPU does; the sequence and its blocks stay as they are."""
+    from engine.memory.block_allocator import BlockTable
+
+    runner = _cpu_runner()
+    runner.model.get_input_embeddings = lambda emb=torch.nn.Embedding(8, 4): emb
+    for token in (-1, 8, 2 ** 31 - 1):
+        table = BlockTable(0, 16, [0], 3)
+        for fields in (dict(last_token_id=token), dict(generated_ids=[1, token])):
+            with pytest.raises(IndexError, match=f"Token id {token} of seq 5"):
+                with torch.inference_mode():
+                    runner.decode_step([SimpleNamespace(seq_id=5, block_table=table, **fields)])
+            assert table.num_tokens == 3
+    with pytest.raises(AttributeError):  # an id it takes: on to the model call, which is a stub here
+        with torch.inference_mode():
+            runner.use_graphs = False
+            runner.decode_step([SimpleNamespace(seq_id=5, block_table=table, last_token_id=7)])
+    assert table.num_tokens == 4
+
+
 def test_free_list_allocator_counts_references():
     from engine.memory.block_allocator import BlockTable, BlockAllocator
 

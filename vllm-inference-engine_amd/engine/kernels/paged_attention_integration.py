@@ -389,8 +389,11 @@ class PagedAttentionContext:
 
     `pool` is any object with per-layer `k_cache`/`v_cache` lists and a
     `device` (the reference's PhysicalBlockPool). Block tables are BlockTable-like
-    objects (`.physical_block_ids`) or plain lists.
+    objects (`.physical_block_ids`) or plain lists. `checked_vocab` is set by a
+    caller that refuses token ids outside [0, checked_vocab) on the host.
     """
+
+    checked_vocab: Optional[int] = None
 
     def __init__(
         self,
@@ -938,10 +941,31 @@ def _stack_takes(self: nn.Module, input_ids, attention_mask, position_ids, past_
             and not any(_has_hooks(layer) for layer in self.layers))
 
 
+def _vocabulary(model: Any) -> Optional[int]:
+    """Rows of the model's input embedding, if that is a plain nn.Embedding."""
+    get = getattr(model, "get_input_embeddings", None)
+    try:
+        emb = get() if get is not None else None
+    except NotImplementedError:  # transformers: the model does not name one
+        emb = None
+    return emb.weight.shape[0] if type(emb) is nn.Embedding else None
+
+
+def _ids_checked(ctx: Any, emb: nn.Embedding) -> bool:
+    """Whether every token id of the context's steps was checked on the host against emb's rows.
+
+    decode_embed gives an id outside the table a row of NaNs, where the
+    embedding module refuses it: ids that nobody checked go to the module.
+    """
+    checked = getattr(ctx, "checked_vocab", None)
+    return checked is not None and checked <= emb.weight.shape[0]
+
+
 def _plain_embedding_and_rope(self: nn.Module) -> bool:
-    """Whether the base model's embedding and rotary modules are the plain ones decode_embed computes."""
+    """Whether decode_embed computes what the base model's embedding and rotary modules would."""
     emb, rope = self.embed_tokens, self.rotary_emb
     return (type(emb) is nn.Embedding and emb.max_norm is None and not _has_hooks(emb)
+            and _ids_checked(self._paged_stack_context, emb)
             and emb.weight.is_cuda and emb.weight.dtype == torch.float16
             and emb.weight.is_contiguous() and emb.weight.data_ptr() % 16 == 0
             and type(rope).__name__ == "Qwen2RotaryEmbedding" and not _has_hooks(rope)
@@ -1171,6 +1195,7 @@ class _DecodeGraph:
         self.lens = self.dev_in[2].view(torch.int32)[:batch]
         self.ctx = PagedAttentionContext.from_device(runner.pool, self.tables, self.lens,
                                                      runner.block_size)
+        self.ctx.checked_vocab = _vocabulary(runner.model)  # decode_step refuses other ids
         self.runner = runner
         self.graph: Optional[torch.cuda.CUDAGraph] = None
         self.logits: Optional[torch.Tensor] = None
@@ -1473,6 +1498,7 @@ class KernelPagedManualDecode:
         if not self._grad_probed:
             self._grad_probed = True
             assert not torch.is_grad_enabled(), "decode_step must run under torch.inference_mode()"
+        vocab = _vocabulary(self.model)
         seq_lens: List[int] = []
         tables: List[Any] = []
         last_tokens: List[int] = []
@@ -1489,16 +1515,20 @@ class KernelPagedManualDecode:
                 raise AssertionError(f"Decode write for seq {_seq_field(seq, 'seq_id', '?')} would "
                                      f"modify shared block {wid} with ref_count "
                                      f"{allocator.ref_counts[wid]}.")
-            bt.num_tokens += 1
-            seq_lens.append(bt.num_tokens)
-            tables.append(bt)
             last = _seq_field(seq, "last_token_id")
             if last is None:
                 gen = _seq_field(seq, "generated_ids")
                 if not gen:
                     raise ValueError("Sequence must provide last_token_id or non-empty generated_ids.")
                 last = gen[-1]
-            last_tokens.append(int(last))
+            last = int(last)
+            if vocab is not None and not 0 <= last < vocab:
+                raise IndexError(f"Token id {last} of seq {_seq_field(seq, 'seq_id', '?')} is outside "
+                                 f"the embedding's {vocab} rows.")
+            bt.num_tokens += 1
+            seq_lens.append(bt.num_tokens)
+            tables.append(bt)
+            last_tokens.append(last)
         if self.use_graphs:
             rows = [bt.physical_block_ids for bt in tables]
             width = max(64, -(-max(len(r) for r in rows) // 64) * 64)
@@ -1510,6 +1540,7 @@ class KernelPagedManualDecode:
             position_ids = torch.tensor([[L - 1] for L in seq_lens], dtype=torch.long,
                                         device=self.device)
             ctx = PagedAttentionContext(self.pool, tables, seq_lens, self.block_size, True)
+            ctx.checked_vocab = vocab
             with patch_paged_attention(self.model, ctx, fuse_layers=self.fuse_layers):
                 out = self.model(input_ids=input_ids, position_ids=position_ids, use_cache=False)
             logits = out.logits[:, -1, :]
