@@ -83,6 +83,21 @@ def test_norm_and_swiglu(cuda_device, rows, n, k):
     _within(act, want, bound + want.abs() * 2.0 ** -21, 1.0)
 
 
+def test_normed_values_up_to_the_largest_fp16(cuda_device):
+    """A normed value that fp16 holds is not an infinity on the way, whatever the row's scale."""
+    rows, n, k = 33, 32, 96
+    x = torch.zeros(rows, k, device=cuda_device, dtype=torch.float16)
+    x[:, 0] = torch.logspace(-1, 1, rows, base=2.0, device=cuda_device).half()
+    gain = torch.full((k,), 6600.0, device=cuda_device).half()  # times sqrt(96): 64666
+    w = (torch.rand(n, k, device=cuda_device) * 2.0 ** -8).half()
+    got = decode_linear(pack_rows(x), pack_weight(w), norm=(gain, EPS), packed=False)
+    xd = x.double()
+    normed = xd * torch.rsqrt(xd.square().mean(1, keepdim=True) + EPS) * gain.double()
+    assert normed.max() < 65504
+    want = normed @ w.double().t()
+    _within(got, want, want.abs(), 2.0 ** -11 + (k + 8) * 2.0 ** -24)
+
+
 def test_sums_of_the_previous_launch_feed_the_norm(cuda_device):
     """A residual row written by one launch is normalised by the next from its partial sums."""
     x, w, g = _data(37, 896, 896, cuda_device, 3)

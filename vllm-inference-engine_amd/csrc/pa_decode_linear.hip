@@ -29,7 +29,7 @@
 //     (ss_out), so the next launch adds a row's few dozen partial sums, loaded
 //     ahead of the fragments, instead of reading the row twice. The scale
 //     rsqrt(mean + eps) is split into a power of two, applied to the fp16
-//     values exactly, and a factor in [0.75, 1.5) applied to the fp32 sums: the
+//     values exactly, and a factor in [1, 2) applied to the fp32 sums: the
 //     product's operand fp16(x * 2^e * weight) is rounded once, where the
 //     unfused norm rounds twice.
 //
@@ -146,7 +146,8 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
 #pragma unroll
       for (int p = 0; p < PARTS; ++p) tot += s_ss[p * ROWS + t * 16 + row];
       const float inv = rsqrtf(tot * a.inv_k + a.eps);
-      const uint32_t e = (__builtin_bit_cast(uint32_t, inv) + 0x400000u) & 0x7f800000u;
+      // Rounded down: the fp16 operand never exceeds the normed value it stands for.
+      const uint32_t e = __builtin_bit_cast(uint32_t, inv) & 0x7f800000u;
       const float p2 = fminf(fmaxf(__builtin_bit_cast(float, e), 0x1p-24f), 0x1p15f);  // fp16's range
       pow2[t] = (f16)p2;
       rest[t] = inv / p2;
