@@ -4,8 +4,8 @@ Compiles every HIP source under csrc/ with hipcc for gfx950 and links them into
 engine/kernels/libpa_gfx950.so, next to the ctypes loader that opens it, and the
 benchmark's read-bandwidth probes (probes/bw_probe.hip) into
 probes/libbw_probe_gfx950.so. The module that calls the library with torch
-tensors (host/pa_host.cpp, host code only) becomes engine/kernels/_pa_host.so,
-linked against the library. Object files go to _build/ at the repository root. Run directly
+tensors (host/pa_host.cpp, host code only) becomes engine/kernels/_pa_host.so
+(not linked against the library: the loader binds it to the one it opened). Object files go to _build/ at the repository root. Run directly
 (``python vllm-inference-engine_amd/build.py``) or through
 ``__graft_entry__.build()``.
 """
@@ -104,9 +104,8 @@ def _link_host(obj: Path) -> None:
     from torch.utils.cpp_extension import library_paths
 
     tmp = HOST_MODULE.with_suffix(".so.tmp")
-    cmd = ["g++", "-shared", str(obj), f"-L{LIB_PATH.parent}", f"-l:{LIB_PATH.name}",
-           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
-           "-Wl,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined", "-o", str(tmp)]
+    cmd = ["g++", "-shared", str(obj), *(f"-L{p}" for p in library_paths()), "-ltorch_python",
+           "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,--allow-shlib-undefined", "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link of {HOST_MODULE.name} failed:\n{proc.stdout}\n{proc.stderr}")

@@ -128,10 +128,13 @@ _host = None
 
 
 def host():
-    """The module that calls the library with torch tensors in native code (host/pa_host.cpp)."""
+    """The module that calls the library with torch tensors in native code (host/pa_host.cpp).
+
+    It calls the library that load() opened, by the addresses given to it here.
+    """
     global _host
     if _host is None:
-        load()
+        lib = load()
         path = LIB_PATH.with_name("_pa_host.so")
         if not path.exists():
             raise NativeLibraryError(
@@ -139,6 +142,8 @@ def host():
         spec = importlib.util.spec_from_file_location("_pa_host", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                     for name in module.CALLS})
         _host = module
     return _host
 

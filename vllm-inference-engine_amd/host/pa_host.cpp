@@ -14,6 +14,9 @@
 // refuses or copies, a tensor subclass or a functorch wrapper, or a workspace
 // too small. The Python entry point then runs its own checks, with its own
 // errors, and its own call.
+//
+// The module is not linked against the library: bind() is given the addresses
+// of the library the process has loaded, whatever file that is.
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
@@ -25,6 +28,27 @@
 namespace {
 
 using at::Tensor;
+
+#define PA_HOST_CALLS(X)                    \
+  X(pa_decode_batched_workspace_bytes)      \
+  X(pa_decode_rope_batched_workspace_bytes) \
+  X(pa_decode_batched_f16)                  \
+  X(pa_decode_kv_write_batched_f16)         \
+  X(pa_decode_rope_batched_f16)
+
+// The loaded library's entry points (bind).
+struct Api {
+#define PA_HOST_MEMBER(name) decltype(&::name) name;
+  PA_HOST_CALLS(PA_HOST_MEMBER)
+#undef PA_HOST_MEMBER
+} api;
+
+void bind(const py::dict& addresses) {
+#define PA_HOST_BIND(name) \
+  api.name = reinterpret_cast<decltype(&::name)>(addresses[#name].cast<uintptr_t>());
+  PA_HOST_CALLS(PA_HOST_BIND)
+#undef PA_HOST_BIND
+}
 
 // Plain strided CUDA tensors of one type on one device.
 bool plain(const Tensor& t, c10::ScalarType type, c10::Device dev) {
@@ -120,7 +144,7 @@ py::object decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
   int64_t qs[3];
   if (!c.fill(q, k, v, bt, lens) || q.dim() != 3 || !rows3(q, c.n, c.hq, c.d, qs) || !rows16(q, qs))
     return py::none();
-  const size_t need = pa_decode_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
+  const size_t need = api.pa_decode_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
   void* wp;
   if (!workspace(ws, q.device(), need, wp)) return py::none();
   const Tensor out = at::empty_like(q);
@@ -128,7 +152,7 @@ py::object decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
   int status;
   {
     py::gil_scoped_release release;
-    status = pa_decode_batched_f16(q.data_ptr(), qs, k.data_ptr(), c.ks, v.data_ptr(), c.vs,
+    status = api.pa_decode_batched_f16(q.data_ptr(), qs, k.data_ptr(), c.ks, v.data_ptr(), c.vs,
                                    (const int32_t*)bt.data_ptr(), c.bts,
                                    (const int32_t*)lens.data_ptr(), out.data_ptr(), os, c.n, c.hq,
                                    c.hkv, c.d, c.bs, c.blocks, c.width, (float)scale, wp, need,
@@ -147,7 +171,7 @@ py::object kv_write_decode(const Tensor& q, const Tensor& key, const Tensor& val
       !rows3(key, c.n, c.hkv, c.d, ys) || !rows16(key, ys) || !rows3(value, c.n, c.hkv, c.d, zs) ||
       !rows16(value, zs))
     return py::none();
-  const size_t need = pa_decode_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
+  const size_t need = api.pa_decode_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
   void* wp;
   if (!workspace(ws, q.device(), need, wp)) return py::none();
   const Tensor out = at::empty({c.n, c.hq, c.d}, q.options());
@@ -155,7 +179,7 @@ py::object kv_write_decode(const Tensor& q, const Tensor& key, const Tensor& val
   int status;
   {
     py::gil_scoped_release release;
-    status = pa_decode_kv_write_batched_f16(
+    status = api.pa_decode_kv_write_batched_f16(
         q.data_ptr(), qs, key.data_ptr(), ys, value.data_ptr(), zs, k.data_ptr(), c.ks,
         v.data_ptr(), c.vs, (const int32_t*)bt.data_ptr(), c.bts, (const int32_t*)lens.data_ptr(),
         out.data_ptr(), os, c.n, c.hq, c.hkv, c.d, c.bs, c.blocks, c.width, (float)scale, wp, need,
@@ -175,7 +199,7 @@ py::object rope_decode(const Tensor& q, const Tensor& key, const Tensor& value, 
       !rows3(key, c.n, c.hkv, c.d, ys) || !rows3(value, c.n, c.hkv, c.d, zs) ||
       !rows2(cos, c.n, c.d, cs) || !rows2(sin, c.n, c.d, ss))
     return py::none();
-  const size_t need = pa_decode_rope_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
+  const size_t need = api.pa_decode_rope_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
   void* wp;
   if (!workspace(ws, q.device(), need, wp)) return py::none();
   const Tensor out = at::empty({c.n, c.hq, c.d}, q.options());
@@ -183,7 +207,7 @@ py::object rope_decode(const Tensor& q, const Tensor& key, const Tensor& value, 
   int status;
   {
     py::gil_scoped_release release;
-    status = pa_decode_rope_batched_f16(
+    status = api.pa_decode_rope_batched_f16(
         q.data_ptr(), qs, key.data_ptr(), ys, value.data_ptr(), zs, cos.data_ptr(), cs,
         sin.data_ptr(), ss, k.data_ptr(), c.ks, v.data_ptr(), c.vs, (const int32_t*)bt.data_ptr(),
         c.bts, (const int32_t*)lens.data_ptr(), out.data_ptr(), os, c.n, c.hq, c.hkv, c.d, c.bs,
@@ -195,6 +219,12 @@ py::object rope_decode(const Tensor& q, const Tensor& key, const Tensor& value, 
 }  // namespace
 
 PYBIND11_MODULE(_pa_host, m) {
+  py::list calls;
+#define PA_HOST_NAME(name) calls.append(#name);
+  PA_HOST_CALLS(PA_HOST_NAME)
+#undef PA_HOST_NAME
+  m.attr("CALLS") = py::tuple(calls);
+  m.def("bind", &bind);
   m.def("decode", &decode);
   m.def("kv_write_decode", &kv_write_decode);
   m.def("rope_decode", &rope_decode);
