@@ -59,7 +59,8 @@ enum {
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
  * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
  * 16: pa_decode_embed_f16; 17: pa_greedy_f16; 18:
- * pa_decode_rope_prefetch_f16). */
+ * pa_decode_rope_prefetch_f16). pa_abi_version returns the library's. */
+#define PA_ABI_VERSION 18
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */

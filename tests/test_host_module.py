@@ -30,3 +30,16 @@ def test_the_module_calls_the_library_that_is_loaded(tmp_path):
                "print('another.so' in maps, '_pa_host.so' in maps, 'libpa_gfx950.so' in maps)\n"
                "print(len(m.CALLS))", tmp_path)
     assert out.split() == ["True", "True", "False", "5"]
+
+
+def test_a_stale_module_is_refused(tmp_path):
+    """Built before the library's interface last changed: refused as a stale library is."""
+    shutil.copy(_native.LIB_PATH, tmp_path / "another.so")
+    shutil.copy(_native.LIB_PATH.with_name("_pa_host.so"), tmp_path / "_pa_host.so")
+    out = _run("_native.load()\n"
+               "_native.ABI_VERSION += 1\n"
+               "try:\n"
+               "    _native.host()\n"
+               "except _native.NativeLibraryError as e:\n"
+               "    print(e)", tmp_path)
+    assert f"_pa_host.so has ABI {_native.ABI_VERSION}, the bindings expect" in out

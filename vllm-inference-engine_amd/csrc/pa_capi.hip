@@ -427,7 +427,7 @@ using namespace pa;
 
 extern "C" {
 
-int pa_abi_version(void) { return 18; }
+int pa_abi_version(void) { return PA_ABI_VERSION; }
 
 const char* pa_last_error(void) { return g_error.c_str(); }
 

@@ -142,6 +142,10 @@ def host():
         spec = importlib.util.spec_from_file_location("_pa_host", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        ver = getattr(module, "ABI_VERSION", None)
+        if ver != ABI_VERSION:
+            raise NativeLibraryError(
+                f"{path} has ABI {ver}, the bindings expect {ABI_VERSION}; rebuild it")
         module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
                      for name in module.CALLS})
         _host = module

@@ -223,6 +223,7 @@ PYBIND11_MODULE(_pa_host, m) {
 #define PA_HOST_NAME(name) calls.append(#name);
   PA_HOST_CALLS(PA_HOST_NAME)
 #undef PA_HOST_NAME
+  m.attr("ABI_VERSION") = PA_ABI_VERSION;  // of the argument lists compiled in here
   m.attr("CALLS") = py::tuple(calls);
   m.def("bind", &bind);
   m.def("decode", &decode);
