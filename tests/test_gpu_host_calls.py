@@ -99,6 +99,38 @@ def test_refusals_are_the_python_checks(cuda_device, name):
     assert empty.shape == (0, HQ, D)
 
 
+class _Marked(torch.Tensor):
+    """A subclass with __torch_function__ alone: no dispatch key tells it from a plain tensor."""
+
+
+@pytest.mark.parametrize("name", ["decode", "kv_write_decode", "rope_decode"])
+def test_subclasses_and_modes_take_the_python_path(cuda_device, monkeypatch, name):
+    t, pools, tables, lens = _tensors(cuda_device, "dense")
+    want = _calls(t, pools, tables, lens, name)
+    native, taken = _native.direct, []
+
+    def watched(*args):
+        out = native(*args)
+        taken.append(out is not None)
+        return out
+
+    monkeypatch.setattr(_native, "direct", watched)
+    got = _calls((t[0].as_subclass(_Marked), *t[1:]), pools, tables, lens, name)
+    assert type(got) is (_Marked if name == "decode" else torch.Tensor)  # empty_like keeps the type
+    assert torch.equal(got.as_subclass(torch.Tensor), want)
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert torch.equal(_calls(t, pools, tables, lens, name), want)
+    assert taken == [False, False]
+    parameter = torch.nn.Parameter(t[0], requires_grad=False)
+    assert torch.equal(_calls((parameter, *t[1:]), pools, tables, lens, name), want)
+    assert taken[-1]
+
+
 def test_a_second_stream_gets_its_own_workspace(cuda_device):
     t, pools, tables, lens = _tensors(cuda_device, "dense")
     want = _calls(t, pools, tables, lens, "decode")

@@ -166,10 +166,7 @@ def direct(name: str, first: torch.Tensor, *args):
     buf = _workspaces.get((index, stream, WS_DECODE))
     if buf is None:
         return None
-    try:
-        return getattr(_host or host(), name)(first, *args, buf, stream)
-    except TypeError:  # something that is not a tensor: the caller's checks say what
-        return None
+    return getattr(_host or host(), name)(first, *args, buf, stream)
 
 
 def i64_array(values) -> ctypes.Array:

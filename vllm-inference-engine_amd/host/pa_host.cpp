@@ -11,16 +11,19 @@
 // Each function launches the call it is given, or returns None without having
 // done anything when something about it is not plain: another device than the
 // current one, a type, shape, alignment or stride the Python entry point
-// refuses or copies, a tensor subclass or a functorch wrapper, or a workspace
-// too small. The Python entry point then runs its own checks, with its own
+// refuses or copies, a tensor subclass, a functorch wrapper, an active
+// __torch_function__ or dispatch mode, or a workspace too small. The Python entry point then runs its own checks, with its own
 // errors, and its own call.
 //
 // The module is not linked against the library: bind() is given the addresses
 // of the library the process has loaded, whatever file that is.
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include "paged_attention.h"
@@ -48,6 +51,19 @@ void bind(const py::dict& addresses) {
   api.name = reinterpret_cast<decltype(&::name)>(addresses[#name].cast<uintptr_t>());
   PA_HOST_CALLS(PA_HOST_BIND)
 #undef PA_HOST_BIND
+}
+
+// The tensors of plain torch.Tensor (or Parameter) objects, with no mode active
+// that intercepts torch calls.
+template <size_t N>
+bool unpack(const py::handle (&objects)[N], const Tensor* (&tensors)[N]) {
+  if (at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return false;
+  for (size_t i = 0; i < N; ++i) {
+    if (!THPVariable_CheckExact(objects[i].ptr())) return false;
+    tensors[i] = &THPVariable_Unpack(objects[i].ptr());
+  }
+  return true;
 }
 
 // Plain strided CUDA tensors of one type on one device.
@@ -138,8 +154,13 @@ py::object done(int status, const Tensor& out) {
   return status == PA_OK ? py::cast(out) : py::object(py::none());
 }
 
-py::object decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& bt,
-                  const Tensor& lens, double scale, const Tensor& ws, int64_t stream) {
+py::object decode(py::handle q_object, py::handle k_object, py::handle v_object, py::handle
+                  bt_object, py::handle lens_object, double scale, py::handle ws_object, int64_t
+                  stream) {
+  const Tensor* t[6];
+  if (!unpack({q_object, k_object, v_object, bt_object, lens_object, ws_object}, t)) return
+               py::none();
+  const Tensor &q = *t[0], &k = *t[1], &v = *t[2], &bt = *t[3], &lens = *t[4], &ws = *t[5];
   Call c;
   int64_t qs[3];
   if (!c.fill(q, k, v, bt, lens) || q.dim() != 3 || !rows3(q, c.n, c.hq, c.d, qs) || !rows16(q, qs))
@@ -161,9 +182,15 @@ py::object decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
   return done(status, out);
 }
 
-py::object kv_write_decode(const Tensor& q, const Tensor& key, const Tensor& value, const Tensor& k,
-                           const Tensor& v, const Tensor& bt, const Tensor& lens, double scale,
-                           const Tensor& ws, int64_t stream) {
+py::object kv_write_decode(py::handle q_object, py::handle key_object, py::handle value_object,
+                           py::handle k_object, py::handle v_object, py::handle bt_object,
+                           py::handle lens_object, double scale, py::handle ws_object, int64_t
+                           stream) {
+  const Tensor* t[8];
+  if (!unpack({q_object, key_object, value_object, k_object, v_object, bt_object, lens_object,
+               ws_object}, t)) return py::none();
+  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &k = *t[3], &v = *t[4], &bt = *t[5], &lens
+               = *t[6], &ws = *t[7];
   Call c;
   int64_t qs[3], ys[3], zs[3];
   if (!c.fill(q, k, v, bt, lens) || !plain(key, at::kHalf, q.device()) ||
@@ -188,9 +215,15 @@ py::object kv_write_decode(const Tensor& q, const Tensor& key, const Tensor& val
   return done(status, out);
 }
 
-py::object rope_decode(const Tensor& q, const Tensor& key, const Tensor& value, const Tensor& cos,
-                       const Tensor& sin, const Tensor& k, const Tensor& v, const Tensor& bt,
-                       const Tensor& lens, double scale, const Tensor& ws, int64_t stream) {
+py::object rope_decode(py::handle q_object, py::handle key_object, py::handle value_object,
+                       py::handle cos_object, py::handle sin_object, py::handle k_object, py::handle
+                       v_object, py::handle bt_object, py::handle lens_object, double scale,
+                       py::handle ws_object, int64_t stream) {
+  const Tensor* t[10];
+  if (!unpack({q_object, key_object, value_object, cos_object, sin_object, k_object, v_object,
+               bt_object, lens_object, ws_object}, t)) return py::none();
+  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &cos = *t[3], &sin = *t[4], &k = *t[5], &v
+               = *t[6], &bt = *t[7], &lens = *t[8], &ws = *t[9];
   Call c;
   int64_t qs[3], ys[3], zs[3], cs[2], ss[2];
   if (!c.fill(q, k, v, bt, lens) || !plain(key, at::kHalf, q.device()) ||
