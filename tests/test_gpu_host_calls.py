@@ -6,6 +6,8 @@ other devices and types, errors) behaves as the Python path alone does.
 """
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -129,6 +131,30 @@ def test_subclasses_and_modes_take_the_python_path(cuda_device, monkeypatch, nam
     parameter = torch.nn.Parameter(t[0], requires_grad=False)
     assert torch.equal(_calls((parameter, *t[1:]), pools, tables, lens, name), want)
     assert taken[-1]
+
+
+# The library's status for a call it refuses before any launch, and for a HIP error.
+@pytest.mark.parametrize("status", [_native.PA_ERR_ARG, _native.PA_ERR_HIP])
+def test_hip_errors_are_raised_once(cuda_device, status):
+    """A refused call is the Python path's to explain; a HIP error is not tried a second time."""
+    t, pools, tables, lens = _tensors(cuda_device, "dense")
+    want = _calls(t, pools, tables, lens, "decode")
+    calls = []
+    failing = ctypes.CFUNCTYPE(ctypes.c_int, *_native.SIGNATURES["pa_decode_batched_f16"][1])(
+        lambda *a: calls.append(1) or status)
+    module, lib = _native.host(), _native.load()
+    addresses = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in module.CALLS}
+    try:
+        module.bind(dict(addresses, pa_decode_batched_f16=ctypes.cast(failing,
+                                                                      ctypes.c_void_p).value))
+        if status == _native.PA_ERR_HIP:
+            with pytest.raises(_native.NativeLibraryError, match=f"status {status}"):
+                _calls(t, pools, tables, lens, "decode")
+        else:
+            assert torch.equal(_calls(t, pools, tables, lens, "decode"), want)
+    finally:
+        module.bind(addresses)
+    assert calls == [1]
 
 
 def test_a_second_stream_gets_its_own_workspace(cuda_device):

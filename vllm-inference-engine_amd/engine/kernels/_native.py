@@ -157,7 +157,7 @@ def direct(name: str, first: torch.Tensor, *args):
 
     None when the call is not a plain one (see host/pa_host.cpp), no
     workspace exists for the stream yet, or first is not on a GPU: the caller
-    then checks and launches it itself.
+    then checks and launches it itself. A HIP error is raised here.
     """
     index = first.get_device()
     if index < 0 or _raw_stream is None:
@@ -166,7 +166,10 @@ def direct(name: str, first: torch.Tensor, *args):
     buf = _workspaces.get((index, stream, WS_DECODE))
     if buf is None:
         return None
-    return getattr(_host or host(), name)(first, *args, buf, stream)
+    out = getattr(_host or host(), name)(first, *args, buf, stream)
+    if type(out) is int:
+        check(out, name)
+    return out
 
 
 def i64_array(values) -> ctypes.Array:

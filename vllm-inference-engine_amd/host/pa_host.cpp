@@ -12,8 +12,10 @@
 // done anything when something about it is not plain: another device than the
 // current one, a type, shape, alignment or stride the Python entry point
 // refuses or copies, a tensor subclass, a functorch wrapper, an active
-// __torch_function__ or dispatch mode, or a workspace too small. The Python entry point then runs its own checks, with its own
-// errors, and its own call.
+// __torch_function__ or dispatch mode, or a workspace too small. The Python entry
+// point then runs its own checks, with its own errors, and its own call. Where the
+// library reports a HIP error, the status is returned for the caller to raise: the
+// call was made, or the error is an earlier one that only this report tells of.
 //
 // The module is not linked against the library: bind() is given the addresses
 // of the library the process has loaded, whatever file that is.
@@ -31,6 +33,7 @@
 namespace {
 
 using at::Tensor;
+using Obj = py::handle;
 
 #define PA_HOST_CALLS(X)                    \
   X(pa_decode_batched_workspace_bytes)      \
@@ -56,7 +59,7 @@ void bind(const py::dict& addresses) {
 // The tensors of plain torch.Tensor (or Parameter) objects, with no mode active
 // that intercepts torch calls.
 template <size_t N>
-bool unpack(const py::handle (&objects)[N], const Tensor* (&tensors)[N]) {
+bool unpack(const Obj (&objects)[N], const Tensor* (&tensors)[N]) {
   if (at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set())
     return false;
   for (size_t i = 0; i < N; ++i) {
@@ -151,15 +154,14 @@ bool workspace(const Tensor& ws, c10::Device dev, size_t need, void*& ptr) {
 }
 
 py::object done(int status, const Tensor& out) {
-  return status == PA_OK ? py::cast(out) : py::object(py::none());
+  if (status == PA_OK) return py::cast(out);
+  return status == PA_ERR_HIP ? py::object(py::int_(status)) : py::object(py::none());
 }
 
-py::object decode(py::handle q_object, py::handle k_object, py::handle v_object, py::handle
-                  bt_object, py::handle lens_object, double scale, py::handle ws_object, int64_t
-                  stream) {
+py::object decode(Obj q_, Obj k_, Obj v_, Obj bt_, Obj lens_, double scale, Obj ws_,
+                  int64_t stream) {
   const Tensor* t[6];
-  if (!unpack({q_object, k_object, v_object, bt_object, lens_object, ws_object}, t)) return
-               py::none();
+  if (!unpack({q_, k_, v_, bt_, lens_, ws_}, t)) return py::none();
   const Tensor &q = *t[0], &k = *t[1], &v = *t[2], &bt = *t[3], &lens = *t[4], &ws = *t[5];
   Call c;
   int64_t qs[3];
@@ -182,15 +184,12 @@ py::object decode(py::handle q_object, py::handle k_object, py::handle v_object,
   return done(status, out);
 }
 
-py::object kv_write_decode(py::handle q_object, py::handle key_object, py::handle value_object,
-                           py::handle k_object, py::handle v_object, py::handle bt_object,
-                           py::handle lens_object, double scale, py::handle ws_object, int64_t
-                           stream) {
+py::object kv_write_decode(Obj q_, Obj key_, Obj value_, Obj k_, Obj v_, Obj bt_, Obj lens_,
+                           double scale, Obj ws_, int64_t stream) {
   const Tensor* t[8];
-  if (!unpack({q_object, key_object, value_object, k_object, v_object, bt_object, lens_object,
-               ws_object}, t)) return py::none();
-  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &k = *t[3], &v = *t[4], &bt = *t[5], &lens
-               = *t[6], &ws = *t[7];
+  if (!unpack({q_, key_, value_, k_, v_, bt_, lens_, ws_}, t)) return py::none();
+  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &k = *t[3], &v = *t[4], &bt = *t[5],
+               &lens = *t[6], &ws = *t[7];
   Call c;
   int64_t qs[3], ys[3], zs[3];
   if (!c.fill(q, k, v, bt, lens) || !plain(key, at::kHalf, q.device()) ||
@@ -215,15 +214,12 @@ py::object kv_write_decode(py::handle q_object, py::handle key_object, py::handl
   return done(status, out);
 }
 
-py::object rope_decode(py::handle q_object, py::handle key_object, py::handle value_object,
-                       py::handle cos_object, py::handle sin_object, py::handle k_object, py::handle
-                       v_object, py::handle bt_object, py::handle lens_object, double scale,
-                       py::handle ws_object, int64_t stream) {
+py::object rope_decode(Obj q_, Obj key_, Obj value_, Obj cos_, Obj sin_, Obj k_, Obj v_, Obj bt_,
+                       Obj lens_, double scale, Obj ws_, int64_t stream) {
   const Tensor* t[10];
-  if (!unpack({q_object, key_object, value_object, cos_object, sin_object, k_object, v_object,
-               bt_object, lens_object, ws_object}, t)) return py::none();
-  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &cos = *t[3], &sin = *t[4], &k = *t[5], &v
-               = *t[6], &bt = *t[7], &lens = *t[8], &ws = *t[9];
+  if (!unpack({q_, key_, value_, cos_, sin_, k_, v_, bt_, lens_, ws_}, t)) return py::none();
+  const Tensor &q = *t[0], &key = *t[1], &value = *t[2], &cos = *t[3], &sin = *t[4], &k = *t[5],
+               &v = *t[6], &bt = *t[7], &lens = *t[8], &ws = *t[9];
   Call c;
   int64_t qs[3], ys[3], zs[3], cs[2], ss[2];
   if (!c.fill(q, k, v, bt, lens) || !plain(key, at::kHalf, q.device()) ||
@@ -232,7 +228,8 @@ py::object rope_decode(py::handle q_object, py::handle key_object, py::handle va
       !rows3(key, c.n, c.hkv, c.d, ys) || !rows3(value, c.n, c.hkv, c.d, zs) ||
       !rows2(cos, c.n, c.d, cs) || !rows2(sin, c.n, c.d, ss))
     return py::none();
-  const size_t need = api.pa_decode_rope_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
+  const size_t need =
+      api.pa_decode_rope_batched_workspace_bytes(c.n, c.hq, c.hkv, c.d, c.bs, c.width);
   void* wp;
   if (!workspace(ws, q.device(), need, wp)) return py::none();
   const Tensor out = at::empty({c.n, c.hq, c.d}, q.options());
