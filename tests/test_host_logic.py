@@ -102,6 +102,7 @@ def test_runner_refuses_token_ids_outside_the_vocabulary():
 
     runner = _cpu_runner()
     runner.model.get_input_embeddings = lambda emb=torch.nn.Embedding(8, 4): emb
+    runner.use_graphs = False
     for token in (-1, 8, 2 ** 31 - 1):
         table = BlockTable(0, 16, [0], 3)
         for fields in (dict(last_token_id=token), dict(generated_ids=[1, token])):
@@ -111,7 +112,6 @@ def test_runner_refuses_token_ids_outside_the_vocabulary():
             assert table.num_tokens == 3
     with pytest.raises(AttributeError):  # an id it takes: on to the model call, which is a stub here
         with torch.inference_mode():
-            runner.use_graphs = False
             runner.decode_step([SimpleNamespace(seq_id=5, block_table=table, last_token_id=7)])
     assert table.num_tokens == 4
 

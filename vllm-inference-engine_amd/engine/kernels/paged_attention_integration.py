@@ -1488,6 +1488,17 @@ class KernelPagedManualDecode:
         return int(tok_margin[0])
 
     # -- decode ------------------------------------------------------------------
+    @staticmethod
+    def _check_ids(seqs: List[Any], tables: List[Any], ids: List[int], vocab: Optional[int]) -> None:
+        """Refuse token ids outside the embedding's rows, with the sequences as they were."""
+        if vocab is None or (min(ids) >= 0 and max(ids) < vocab):
+            return
+        for table in tables:
+            table.num_tokens -= 1
+        seq, i = next((s, i) for s, i in zip(seqs, ids) if not 0 <= i < vocab)
+        raise IndexError(f"Token id {i} of seq {_seq_field(seq, 'seq_id', '?')} is outside the "
+                         f"embedding's {vocab} rows.")
+
     @torch.inference_mode()
     def decode_step(self, seqs: List[Any], allocator: Any = None) -> List[int]:
         """One batched decode step for the running sequences (reference :518-653)."""
@@ -1498,7 +1509,6 @@ class KernelPagedManualDecode:
         if not self._grad_probed:
             self._grad_probed = True
             assert not torch.is_grad_enabled(), "decode_step must run under torch.inference_mode()"
-        vocab = _vocabulary(self.model)
         seq_lens: List[int] = []
         tables: List[Any] = []
         last_tokens: List[int] = []
@@ -1521,21 +1531,21 @@ class KernelPagedManualDecode:
                 if not gen:
                     raise ValueError("Sequence must provide last_token_id or non-empty generated_ids.")
                 last = gen[-1]
-            last = int(last)
-            if vocab is not None and not 0 <= last < vocab:
-                raise IndexError(f"Token id {last} of seq {_seq_field(seq, 'seq_id', '?')} is outside "
-                                 f"the embedding's {vocab} rows.")
             bt.num_tokens += 1
             seq_lens.append(bt.num_tokens)
             tables.append(bt)
-            last_tokens.append(last)
+            last_tokens.append(int(last))
         if self.use_graphs:
             rows = [bt.physical_block_ids for bt in tables]
             width = max(64, -(-max(len(r) for r in rows) // 64) * 64)
             graph = self._decode_graph(n, width)
+            # The table its launches read (and a lookup of the model's takes 9 us per step).
+            self._check_ids(seqs, tables, last_tokens, graph.ctx.checked_vocab)
             graph.load(last_tokens, seq_lens, rows)
             logits = graph.run()
         else:
+            vocab = _vocabulary(self.model)
+            self._check_ids(seqs, tables, last_tokens, vocab)
             input_ids = torch.tensor(last_tokens, dtype=torch.long, device=self.device).unsqueeze(1)
             position_ids = torch.tensor([[L - 1] for L in seq_lens], dtype=torch.long,
                                         device=self.device)
