@@ -59,8 +59,9 @@ enum {
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
  * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
  * 16: pa_decode_embed_f16; 17: pa_greedy_f16; 18:
- * pa_decode_rope_prefetch_f16). pa_abi_version returns the library's. */
-#define PA_ABI_VERSION 18
+ * pa_decode_rope_prefetch_f16; 19: weight_row_stride of pa_decode_linear_f16).
+ * pa_abi_version returns the library's. */
+#define PA_ABI_VERSION 19
 PA_API int pa_abi_version(void);
 
 /* Message of the last failed call on this thread ("" after a success). */
@@ -410,8 +411,9 @@ PA_API int pa_greedy_f16(const void* logits, int64_t row_stride, int rows, int v
  * to row_sums[rows].
  *
  * pa_decode_linear_f16: y = epilogue(norm(x) W^T), fp32 accumulation. x is
- * packed (x_row_stride 0) or row-major; weight [n, k] is packed. With
- * norm_weight, x (packed) is first RMS-normalised: scaled by norm_weight and by
+ * packed (x_row_stride 0) or row-major; weight [n, k] is packed (weight_row_stride
+ * 0) or, without norm_weight and silu_pairs, row-major. With norm_weight, x
+ * (packed) is first RMS-normalised: scaled by norm_weight and by
  * rsqrt(sum / k + eps), sum being the row's num_row_sums partial sums of
  * squares row_sums[num_row_sums][rows]. Then bias[n] and the packed residual
  * [rows, n] are added in fp32 (either may be NULL). With silu_pairs, weight
@@ -434,11 +436,11 @@ PA_API int pa_decode_embed_f16(const int64_t* ids, const int64_t* positions, con
                                float scaling, int head_dim, void* packed, float* row_sums,
                                void* cos, void* sin, int rows, void* stream);
 PA_API int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,
-                                const void* norm_weight, const float* row_sums,
-                                int num_row_sums, float eps, const void* bias,
-                                const void* residual, void* y, int64_t y_row_stride,
-                                float* row_sums_out, int rows, int n, int k, int silu_pairs,
-                                void* stream);
+                                int64_t weight_row_stride, const void* norm_weight,
+                                const float* row_sums, int num_row_sums, float eps,
+                                const void* bias, const void* residual, void* y,
+                                int64_t y_row_stride, float* row_sums_out, int rows, int n,
+                                int k, int silu_pairs, void* stream);
 
 /*
  * Batched decode attention that allocates nothing. No counterpart in the

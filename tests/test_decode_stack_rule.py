@@ -11,6 +11,7 @@ from engine.kernels.paged_attention_integration import (
     PagedAttentionContext,
     _ids_checked,
     _stack_takes,
+    _weights_readable,
 )
 
 
@@ -97,3 +98,38 @@ def test_only_ids_checked_against_the_table_skip_the_embedding_module():
     for checked, taken in ((8, True), (5, True), (9, False)):
         ctx.checked_vocab = checked
         assert _ids_checked(ctx, emb) == taken
+
+
+def test_weights_the_kernels_cannot_read_take_the_layers():
+    """The parameters that the stack reads in place: another type, shape, stride or alignment."""
+    half = dict(dtype=torch.float16)
+
+    def layer():
+        linear = lambda n, k: SimpleNamespace(weight=torch.zeros(n, k, **half), bias=None,  # noqa: E731
+                                              out_features=n)
+        norm = lambda: SimpleNamespace(weight=torch.zeros(64, **half))  # noqa: E731
+        return SimpleNamespace(
+            self_attn=SimpleNamespace(o_proj=linear(64, 32), q_proj=linear(32, 64)),
+            mlp=SimpleNamespace(down_proj=linear(64, 96)), input_layernorm=norm(),
+            post_attention_layernorm=norm(),
+            _pa_packed=(torch.zeros(4, 2, 4, 16, 8, **half), torch.zeros(12, 2, 4, 16, 8, **half)))
+
+    assert _weights_readable(layer())
+    wide, odd = torch.zeros(64, 40, **half), torch.zeros(64 * 32 + 4, **half)
+    m = layer()
+    m.self_attn.o_proj.weight = wide[:, :32]
+    assert _weights_readable(m)
+    for name, weight in (("o_proj", torch.zeros(64, 32)), ("o_proj", torch.zeros(64, 64, **half)),
+                         ("o_proj", torch.zeros(32, 64, **half).t()),
+                         ("o_proj", torch.zeros(64, 36, **half)[:, :32]),
+                         ("o_proj", odd[4:].view(64, 32)),
+                         ("down_proj", torch.zeros(64, 64, **half))):
+        m = layer()
+        getattr(m.self_attn if name == "o_proj" else m.mlp, name).weight = weight
+        assert not _weights_readable(m)
+    m = layer()
+    m.self_attn.o_proj.bias = torch.zeros(64)
+    assert not _weights_readable(m)
+    m = layer()
+    m.input_layernorm.weight = torch.zeros(65, **half)[1:]
+    assert not _weights_readable(m)

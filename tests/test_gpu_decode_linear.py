@@ -57,6 +57,32 @@ def test_linear_with_bias_residual_and_sums(cuda_device, rows, n, k):
     assert out.sums.shape == (n // 16, rows)
 
 
+# Row-major weights, loaded four K steps at a time: K of fewer steps than wavefronts, ranges that end
+# inside a block of four, both wavefront counts; column tiles (71 and 72 of them) and row tiles that
+# leave remainders for every tile shape; rows of a wider buffer.
+@pytest.mark.parametrize("rows", [1, 17, 50, 100, 128, 241, 256])
+@pytest.mark.parametrize("n,k", [(32, 32), (1136, 96), (1152, 896), (1136, 2336), (896, 4864)])
+def test_row_major_weights(cuda_device, rows, n, k):
+    x, w, g = _data(rows, n, k, cuda_device, rows * 13 + n + k)
+    wide = torch.full((n, k + 24), float("nan"), device=cuda_device).half()
+    wide[:, :k] = w
+    bias = torch.randn(n, generator=g, device=cuda_device).half()
+    want = x.double() @ w.double().t() + bias.double()
+    terms = x.double().abs() @ w.double().abs().t() + bias.double().abs()
+    got = decode_linear(x, w, bias=bias, packed=False)
+    _within(got, want, terms, k * 2.0 ** -24)
+    for again in (decode_linear(pack_rows(x), w, bias=bias, packed=False),
+                  decode_linear(x, wide[:, :k], bias=bias, packed=False)):
+        assert torch.equal(got, again)
+    if n % 32:
+        return
+    res = torch.randn(rows, n, generator=g, device=cuda_device).half()
+    out = decode_linear(x, w, bias=bias, residual=pack_rows(res), sums=True)
+    _within(out.unpack(), want + res.double(), terms + res.double().abs(), (k + 1) * 2.0 ** -24)
+    squares = out.unpack().double().square()
+    assert torch.allclose(out.sums.double().sum(0), squares.sum(1), rtol=n * 2.0 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("rows", [1, 16, 31, 48, 64, 100, 128, 256])
 @pytest.mark.parametrize("n,k", [(32, 64), (1152, 896), (224, 2304)])
 def test_norm_and_swiglu(cuda_device, rows, n, k):
@@ -155,6 +181,45 @@ def test_stack_and_layer_paths_agree(cuda_device):
     diff = (logits[0] - logits[1]).norm() / logits[1].norm()
     print(f"[decode-linear] stack against layers: {diff.item():.2e}", flush=True)
     assert diff <= 20 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("use_graphs", [False, True])
+def test_o_and_down_follow_their_parameters(cuda_device, use_graphs):
+    """In-place changes of the two weights that are not merged with others reach the next step, also
+    through a graph captured before, as in the layer path."""
+    from engine import workloads
+    from engine.kernels.paged_attention_integration import KernelPagedManualDecode
+    from engine.memory.block_allocator import BlockTable
+
+    config = dict(vocab_size=512, hidden_size=128, intermediate_size=256, num_hidden_layers=2,
+                  num_attention_heads=4, num_key_value_heads=2, max_position_embeddings=4096,
+                  rope_theta=1e6, tie_word_embeddings=False)
+    with torch.inference_mode():
+        model = workloads.decode_model(cuda_device, 13, config)
+
+        def logits(runner):
+            gen = torch.Generator(device=cuda_device).manual_seed(2)
+            for c in runner.pool.k_cache + runner.pool.v_cache:
+                c.normal_(0, 0.6, generator=gen)
+            seqs = [{"seq_id": i, "block_table": BlockTable(i, 16, [i], 5 + i),
+                     "last_token_id": 7 * i} for i in range(5)]
+            runner.decode_step(seqs)
+            return torch.stack([s["last_logits"] for s in seqs]).float()
+
+        runner = KernelPagedManualDecode(model, num_blocks=8, device=str(cuda_device),
+                                         use_graphs=use_graphs)
+        old = logits(runner)
+        model.model.layers[0].self_attn.o_proj.weight.mul_(-3)
+        model.model.layers[1].mlp.down_proj.weight.data.copy_(
+            model.model.layers[1].mlp.down_proj.weight * 2)
+        new = logits(runner)
+        handle = model.model.layers[0].register_forward_hook(lambda *a: None)  # the layer path
+        want = logits(KernelPagedManualDecode(model, num_blocks=8, device=str(cuda_device),
+                                              use_graphs=False))
+        handle.remove()
+    # Two layers of fp16 activations: some fourteen roundings of 2^-11.
+    assert (new - want).norm() <= 14 * 2.0 ** -11 * want.norm()
+    assert (new - old).norm() >= 0.1 * want.norm()
 
 
 @pytest.mark.parametrize("use_graphs", [False, True])

@@ -1445,7 +1445,7 @@ int pa_decode_embed_f16(const int64_t* ids, const int64_t* positions, const void
 }
 
 int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight,
-                         const void* norm_weight, const float* row_sums, int num_row_sums,
+                         int64_t weight_row_stride, const void* norm_weight, const float* row_sums, int num_row_sums,
                          float eps, const void* bias, const void* residual, void* y,
                          int64_t y_row_stride, float* row_sums_out, int rows, int n, int k,
                          int silu_pairs, void* stream) {
@@ -1466,6 +1466,15 @@ int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight
               "at a 4-element aligned one (0: packed)");
     return PA_ERR_ARG;
   }
+  if (weight_row_stride && (weight_row_stride < k || weight_row_stride % 8)) {
+    set_error("row-major weight rows need at least k elements at an 8-element aligned stride "
+              "(0: packed)");
+    return PA_ERR_ARG;
+  }
+  if (weight_row_stride && (norm_weight || silu_pairs)) {
+    set_error("norm and silu pairs take a packed weight");
+    return PA_ERR_UNSUPPORTED;
+  }
   if ((y_packed || residual) && n % 32) {
     set_error("a packed output or residual needs n to be a multiple of 32");
     return PA_ERR_ARG;
@@ -1480,8 +1489,8 @@ int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight
     return PA_ERR_ARG;
   }
   // Byte offsets inside a tile of rows are 32-bit.
-  if (k > (1 << 25) || x_row_stride > (1 << 24)) {
-    set_error("k %d or the row stride of x exceeds the kernel's 32-bit tile offsets", k);
+  if (k > (1 << 25) || x_row_stride > (1 << 24) || weight_row_stride > (1 << 24)) {
+    set_error("k %d or a row stride exceeds the kernel's 32-bit tile offsets", k);
     return PA_ERR_UNSUPPORTED;
   }
   LinearArgs a{};
@@ -1494,6 +1503,7 @@ int pa_decode_linear_f16(const void* x, int64_t x_row_stride, const void* weight
   a.res = (const f16*)residual;
   a.ss_out = row_sums_out;
   a.ldx = x_row_stride;
+  a.ldw = weight_row_stride;
   a.ldy = y_row_stride;
   a.M = rows;
   a.N = n;

@@ -363,14 +363,14 @@ __host__ __device__ constexpr int record_floats(int D) { return 32 + 16 * D; }
 // w[n, k] over the packed layout below.
 struct LinearArgs {
   const f16* x;    // [M, K] packed, or row-major with row stride ldx
-  const f16* w;    // [N, K] packed (with silu [2 N, K]: gate rows, then up rows)
+  const f16* w;    // [N, K] packed (with silu [2 N, K]: gate rows, then up rows), or row-major
   f16* y;          // [M, N] packed, or row-major with row stride ldy
   const f16* norm;  // RMSNorm weight [K] applied to x, or null
   const float* ss;  // with norm: ss_parts partial sums of squares per row, [ss_parts][M]
   const f16* bias;  // [N] or null
   const f16* res;   // [M, N] packed, added to the product, or null
   float* ss_out;    // per 16-column tile of y its rows' sums of squares, [N / 16][M], or null
-  int64_t ldx, ldy;
+  int64_t ldx, ldy, ldw;  // ldw: row stride of row-major weights, 0: packed
   int M, N, K;
   int mtiles;  // workgroups along M (set at launch)
   int ss_parts, y_packed;

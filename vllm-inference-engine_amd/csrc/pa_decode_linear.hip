@@ -19,6 +19,17 @@
 //     5.4 (down projection 4864 -> 896 at 8 rows) and 16.2 instead of 7.9 us
 //     (128 rows). Weights are packed once; activations are written packed by
 //     the launch that produces them.
+//   * Weights that a program may change in place (o and down, which are not
+//     merged with others) are read where they are, row-major (WROW). A fragment
+//     takes its 8 values of row lane % 16 from every lane; loaded so, 16
+//     neighbouring lanes touch 16 rows. Instead two loads fetch two K steps of a tile,
+//     eight lanes to 128 consecutive bytes of a row, and the wavefront exchanges them
+//     through LDS of its own. Us per launch as below, cold weights and from L2: down at
+//     8 rows packed 5.5 and 4.4, row-major loads 7.8, this 6.2 and 5.2; o 3.2 and 2.9,
+//     3.7, 3.5 and 3.1; at 128 rows down 7.0 and 5.9, 13.4, 7.8 and 6.9, o 3.8 and 3.5,
+//     5.7, 4.3 and 3.9. Four steps at a time, 64 bytes of a row to four lanes and a
+//     transpose in registers: down 6.5 and 5.4, 8.1 and 7.3. A packed copy would be
+//     faster but would not follow the parameter.
 //   * K is split over the workgroup's wavefronts: each loads its own weight
 //     and X fragments straight into registers, DEPTH steps ahead, multiplies,
 //     and the wavefronts' tiles are summed through LDS in wavefront order (the
@@ -50,13 +61,14 @@ using namespace tiles;
 // gate and the up rows of the merged weight) by TM tiles of 16 rows, K split
 // over NW wavefronts. Tiles past the end of N or M repeat the last one and are
 // not stored; K steps past a wavefront's range load zeros (empty resources),
-// so no branch separates the loads.
-template <int NW, int TN, int TM, int DEPTH, bool NORM, bool SILU, bool XPACK>
+// so no branch separates the loads. WROW: row-major weights.
+template <int NW, int TN, int TM, int DEPTH, bool NORM, bool SILU, bool XPACK, bool WROW>
 __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
   constexpr int TO = SILU ? TN / 2 : TN;
   constexpr int ROWS = 16 * TM;
   constexpr int PARTS = 64 * NW / ROWS;  // threads that add one row's partial sums
   static_assert(!SILU || TN % 2 == 0, "a gate tile goes with its up tile");
+  static_assert(!WROW || DEPTH % 2 == 0, "row-major weights come two steps at a time");
   static_assert(PARTS * ROWS == 64 * NW, "threads must split evenly over the rows");
   __shared__ __attribute__((aligned(16))) float s_red[NW * TN * TM * 256];
   __shared__ float s_ss[NORM ? PARTS * ROWS : 1];
@@ -100,7 +112,7 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     const int t = min(o0 + (SILU ? i % TO : i), ntiles - 1) + (SILU && i >= TO ? ntiles : 0);
-    wt[i] = a.w + (int64_t)t * a.K * 16;
+    wt[i] = a.w + (int64_t)t * 16 * (WROW ? a.ldw : a.K);
   }
   const f16* xt[TM];
   uint32_t x_lane[TM];
@@ -116,6 +128,33 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
   }
 
   u32x4 wf[DEPTH][TN], xf[DEPTH][TM], nf[NORM ? DEPTH : 1];
+  // Row-major weights: load j of a pair holds rows 8 (j % 2) + lane / 8 of the tile, piece (8
+  // values of K) lane % 8 of the pair's two steps. In LDS a piece's 16 rows are consecutive,
+  // pieces 32 bytes further apart than they need be, so that neither the stores (two rows by
+  // eight pieces per 16 lanes) nor the loads (16 rows) meet in a bank.
+  constexpr int kPiece = 16 * 16 + 32;
+  constexpr int kTile = 8 * kPiece;
+  constexpr int kEnd = 0x7ff00000;  // past every tile: loads return zero
+  __shared__ __attribute__((aligned(16))) char s_w[WROW ? NW * TN * kTile : 16];
+  const int w_lane = (lane >> 3) * (int)a.ldw * 2 + (lane & 7) * 16;
+  const int w_put = wave * TN * kTile + (lane & 7) * kPiece + (lane >> 3) * 16;
+  const int w_get = wave * TN * kTile + grp * kPiece + row * 16;
+  auto load_rows = [&](int j, int u, const f16* w) {
+    const int pair = u - (j & 1);  // the pair's first step
+    const bool in = pair + ((lane >> 2) & 1) < u1;
+    return __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(w, kEnd), in ? w_lane : kEnd,
+                                                 (j & 1) * 16 * (int)a.ldw + pair * 64, 0);
+  };
+  // The fragments of loads j and j + 1, in place.
+  auto exchange = [&](int j) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      *reinterpret_cast<u32x4*>(&s_w[w_put + i * kTile]) = wf[j][i];
+      *reinterpret_cast<u32x4*>(&s_w[w_put + i * kTile + 8 * 16]) = wf[j + 1][i];
+      wf[j][i] = *reinterpret_cast<const u32x4*>(&s_w[w_get + i * kTile]);
+      wf[j + 1][i] = *reinterpret_cast<const u32x4*>(&s_w[w_get + i * kTile + 4 * kPiece]);
+    }
+  };
   auto load = [&](int j, int u) {
     const int nb = u < u1 ? 0x7fffffff : 0;
 #pragma unroll
@@ -124,7 +163,9 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
                                                        u * (XPACK ? 1024 : 64), 0);
 #pragma unroll
     for (int i = 0; i < TN; ++i)
-      wf[j][i] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(wt[i], nb), lane * 16, u * 1024, 0);
+      wf[j][i] = WROW ? load_rows(j, u, wt[i])
+                      : __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(wt[i], nb), lane * 16,
+                                                              u * 1024, 0);
     if constexpr (NORM)
       nf[j] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(a.norm, nb), grp * 16, u * 64, 0);
   };
@@ -161,6 +202,9 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
     for (int t = 0; t < TM; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   auto product = [&](int j) {
+    if constexpr (WROW) {
+      if (j % 2 == 0) exchange(j);
+    }
     f16x8 xv[TM];
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
@@ -178,7 +222,9 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) {
       product(j);
+      if (WROW && j % 2 == 0) continue;  // the pair's registers are free after its second step
       __builtin_amdgcn_sched_barrier(0);
+      if (WROW) load(j - 1, u + DEPTH + j - 1);
       load(j, u + DEPTH + j);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -261,13 +307,14 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const f16* __restrict__ 
   if (threadIdx.x == 0) ss[m] = part[0] + part[1] + part[2] + part[3];
 }
 
-template <int NW, int TN, int TM, int DEPTH, bool NORM, bool SILU, bool XPACK>
+template <int NW, int TN, int TM, int DEPTH, bool NORM, bool SILU, bool XPACK, bool WROW = false>
 static hipError_t launch_tile(LinearArgs a, hipStream_t s) {
   constexpr int TO = SILU ? TN / 2 : TN;
   a.mtiles = (a.M + 16 * TM - 1) / (16 * TM);
   const int64_t grid = (int64_t)a.mtiles * ((a.N / 16 + TO - 1) / TO);
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
-  decode_linear_kernel<NW, TN, TM, DEPTH, NORM, SILU, XPACK><<<(unsigned)grid, 64 * NW, 0, s>>>(a);
+  decode_linear_kernel<NW, TN, TM, DEPTH, NORM, SILU, XPACK, WROW>
+      <<<(unsigned)grid, 64 * NW, 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -295,8 +342,29 @@ static hipError_t launch_plain(const LinearArgs& a, int cus, hipStream_t s) {
               : launch_tile<4, 2, 2, 7, NORM, false, XPACK>(a, s);
 }
 
+// Row-major weights: as launch_plain, but a long K pays for each weight tile's
+// exchange, so two row tiles share one before two column tiles do (down, us, cold and
+// from L2, 128 rows: 1 x 2 7.8 and 6.9, 2 x 1 9.7 and 9.1, 2 x 2 11.3 and 9.3; o at 128
+// rows 2 x 1 4.3 and 3.9, 1 x 2 4.6 and 4.2).
+template <bool XPACK>
+static hipError_t launch_row(const LinearArgs& a, int cus, hipStream_t s) {
+  const int64_t mt = (a.M + 15) / 16, nt = a.N / 16;
+  const bool wide = a.K > 32 * 4 * 14;
+  if (mt * nt <= cus)
+    return wide ? launch_tile<8, 1, 1, 10, false, false, XPACK, true>(a, s)
+                : launch_tile<4, 1, 1, 8, false, false, XPACK, true>(a, s);
+  if (wide && mt > 1 && (mt + 1) / 2 * nt <= cus)
+    return launch_tile<8, 1, 2, 10, false, false, XPACK, true>(a, s);
+  if (mt == 1 || (!wide && mt * ((nt + 1) / 2) <= cus))
+    return wide ? launch_tile<8, 2, 1, 10, false, false, XPACK, true>(a, s)
+                : launch_tile<4, 2, 1, 8, false, false, XPACK, true>(a, s);
+  return wide ? launch_tile<8, 2, 2, 8, false, false, XPACK, true>(a, s)
+              : launch_tile<4, 2, 2, 8, false, false, XPACK, true>(a, s);
+}
+
 hipError_t launch_decode_linear(const LinearArgs& a, bool x_packed, bool silu, int cus,
                                 hipStream_t s) {
+  if (a.ldw) return x_packed ? launch_row<true>(a, cus, s) : launch_row<false>(a, cus, s);
   if (!silu) {
     if (a.norm) return launch_plain<true, true>(a, cus, s);
     return x_packed ? launch_plain<false, true>(a, cus, s) : launch_plain<false, false>(a, cus, s);

@@ -18,7 +18,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
 LIB_NAME = "libpa_gfx950.so"
 LIB_PATH = Path(__file__).with_name(LIB_NAME)
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 PA_OK = 0
 PA_ERR_ARG = 1
@@ -76,8 +76,8 @@ SIGNATURES: dict[str, tuple] = {
     "pa_pack_rows_f16": (_i32, [_vp, _i64, _vp, _vp, _i32, _i32, _vp]),
     "pa_decode_embed_f16": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _i32, _f32, _i32, _vp, _vp, _vp,
                                    _vp, _i32, _vp]),
-    "pa_decode_linear_f16": (_i32, [_vp, _i64, _vp, _vp, _vp, _i32, _f32, _vp, _vp, _vp, _i64, _vp,
-                                    _i32, _i32, _i32, _i32, _vp]),
+    "pa_decode_linear_f16": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _i32, _f32, _vp, _vp, _vp, _i64,
+                                    _vp, _i32, _i32, _i32, _i32, _vp]),
     "pa_decode_rope_batched_f16": (_i32, [
         _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p, _vp, _i64p,
         _vp, _i64p, _vp, _vp, _i64p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp, _sz,

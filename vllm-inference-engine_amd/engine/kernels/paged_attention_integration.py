@@ -753,7 +753,8 @@ def decode_embed(
 
 def decode_linear(
     x: Union[torch.Tensor, PackedRows],  # rows [rows, k]
-    weight: torch.Tensor,                # pack_weight of [n, k]; with silu of [2 n, k] (gate, up)
+    weight: torch.Tensor,                # pack_weight of [n, k]; with silu of [2 n, k] (gate, up);
+                                         # without norm and silu also [n, k] itself, any row stride
     norm: Optional[Tuple[torch.Tensor, float]] = None,  # RMSNorm weight [k] and eps, for a packed x
     bias: Optional[torch.Tensor] = None,
     residual: Optional[PackedRows] = None,
@@ -766,8 +767,12 @@ def decode_linear(
     Returns PackedRows (with the partial sums of squares a following norm needs,
     if asked) or, with packed=False, a row-major [rows, n] tensor.
     """
-    k = weight.shape[1] * 32
-    n = weight.shape[0] * 16 // (2 if silu else 1)
+    if weight.dim() == 2:
+        (n, k), w_stride = weight.shape, weight.stride(0)
+        assert norm is None and not silu and _packable(weight) and weight.stride(1) == 1
+    else:
+        k, w_stride = weight.shape[1] * 32, 0
+        n = weight.shape[0] * 16 // (2 if silu else 1)
     if isinstance(x, PackedRows):
         xd, x_stride, rows, width = x.data, 0, x.rows, x.width
     else:
@@ -804,8 +809,8 @@ def decode_linear(
     lib = _native.load()
     with _on_device(xd.device):
         status = lib.pa_decode_linear_f16(
-            xd.data_ptr(), x_stride, weight.data_ptr(), ptrs[0], ptrs[1], parts, float(eps), ptrs[2],
-            ptrs[3], y_ptr, y_stride, ptrs[4], rows, n, k, int(silu),
+            xd.data_ptr(), x_stride, weight.data_ptr(), w_stride, ptrs[0], ptrs[1], parts, float(eps),
+            ptrs[2], ptrs[3], y_ptr, y_stride, ptrs[4], rows, n, k, int(silu),
             _native.stream_handle(xd.device))
     _native.check(status, "pa_decode_linear_f16")
     return out
@@ -823,11 +828,11 @@ def prepare_fused_layers(model: nn.Module) -> int:
     """Concatenate each decoder layer's q/k/v and gate/up weights once, for the fused decode path.
 
     The merged copies live on the layer (`_pa_fused`); the model's own modules
-    are left as they are. Where the sizes allow it, all four projections are
-    also kept in the packed layout of the decode-step kernels (`_pa_packed`:
-    q/k/v, o, gate/up, down; fused_decoder_stack_forward). Returns the number of
-    layers prepared. Inference only: the copies do not follow later changes of
-    the weights.
+    are left as they are. Where the sizes allow it, the merged weights are also
+    kept in the packed layout of the decode-step kernels (`_pa_packed`: q/k/v,
+    gate/up; fused_decoder_stack_forward). Returns the number of layers prepared.
+    Inference only: the copies do not follow later changes of the weights; o and
+    down are read from the model's own parameters by every path.
     """
     n = 0
     if not isinstance(model, nn.Module):
@@ -852,7 +857,7 @@ def prepare_fused_layers(model: nn.Module) -> int:
             weights = (m._pa_fused[0], attn.o_proj.weight, m._pa_fused[2], mlp.down_proj.weight)
             if all(w.is_cuda and _packable(w) for w in weights) and \
                     weights[0].shape[1] % 32 == 0 and weights[3].shape[0] % 32 == 0:
-                m._pa_packed = tuple(pack_weight(w) for w in weights)
+                m._pa_packed = (pack_weight(weights[0]), pack_weight(weights[2]))
             n += 1
     return n
 
@@ -975,6 +980,27 @@ def _plain_embedding_and_rope(self: nn.Module) -> bool:
             and rope.inv_freq.is_contiguous())
 
 
+def _readable(t: torch.Tensor, shape: Tuple[int, ...], device: torch.device, align: int) -> bool:
+    """Whether the projection kernels read t where it is: fp16 of that shape, aligned rows."""
+    return (t.device == device and t.dtype == torch.float16 and t.shape == shape
+            and t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1])
+            and t.data_ptr() % align == 0)
+
+
+def _weights_readable(layer: nn.Module) -> bool:
+    """Whether a prepared layer's own parameters, as they now are, suit the fused stack."""
+    attn, mlp = layer.self_attn, layer.mlp
+    qkv, gate_up = layer._pa_packed
+    dev, hidden, inter = qkv.device, qkv.shape[1] * 32, gate_up.shape[0] * 8
+    width = attn.q_proj.out_features
+    bias = attn.o_proj.bias
+    return (_readable(attn.o_proj.weight, (hidden, width), dev, 16)
+            and _readable(mlp.down_proj.weight, (hidden, inter), dev, 16)
+            and (bias is None or _readable(bias, (hidden,), dev, 8))
+            and all(_readable(m.weight, (hidden,), dev, 16)
+                    for m in (layer.input_layernorm, layer.post_attention_layernorm)))
+
+
 def fused_decoder_stack_forward(
     self: nn.Module,
     input_ids: Optional[torch.Tensor] = None,
@@ -992,11 +1018,12 @@ def fused_decoder_stack_forward(
     RoPE, K/V write and paged attention; o + residual; post-attention norm +
     gate/up + SwiGLU; down + residual. Calls that ask for more than a decode
     step's hidden states (masks, caches, hidden-state outputs, tuples), layers with
-    forward hooks and more than DECODE_LINEAR_MAX_ROWS rows take the layers one
-    by one as before.
+    forward hooks, weights the kernels cannot read and more than
+    DECODE_LINEAR_MAX_ROWS rows take the layers one by one as before.
     """
     if not _stack_takes(self, input_ids, attention_mask, position_ids, past_key_values,
-                        inputs_embeds, use_cache, kwargs):
+                        inputs_embeds, use_cache, kwargs) or \
+            not all(_weights_readable(layer) for layer in self.layers):
         return self._orig_stack_forward(input_ids=input_ids, attention_mask=attention_mask,
                                         position_ids=position_ids, past_key_values=past_key_values,
                                         inputs_embeds=inputs_embeds, use_cache=use_cache, **kwargs)
@@ -1017,7 +1044,8 @@ def fused_decoder_stack_forward(
         rows = pack_rows(x.view(b, -1))
     for i, layer in enumerate(layers):
         attn, mlp = layer.self_attn, layer.mlp
-        qkv_w, o_w, gu_w, down_w = layer._pa_packed
+        qkv_w, gu_w = layer._pa_packed
+        o_w, down_w = attn.o_proj.weight, mlp.down_proj.weight
         hd = attn.head_dim
         nq = attn.q_proj.out_features // hd
         nkv = attn.k_proj.out_features // hd
@@ -1029,7 +1057,7 @@ def fused_decoder_stack_forward(
             qkv[:, :nq * hd].view(b, nq, hd), qkv[:, nq * hd:(nq + nkv) * hd].view(b, nkv, hd),
             qkv[:, (nq + nkv) * hd:].view(b, nkv, hd), cos, sin, ctx.pool.k_cache[attn.layer_idx],
             ctx.pool.v_cache[attn.layer_idx], ctx.padded_block_tables, ctx.seq_lens_tensor, scale,
-            prefetch=(o_w, *gu_w.chunk(2), down_w))
+            prefetch=[w for w in (o_w, *gu_w.chunk(2), down_w) if w.is_contiguous()])
         h = decode_linear(o.view(b, nq * hd), o_w, bias=attn.o_proj.bias, residual=rows, sums=True)
         act = decode_linear(h, gu_w, norm=(norm2.weight, norm2.variance_epsilon), silu=True)
         last = i + 1 == len(layers)
