@@ -6,10 +6,12 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from engine.kernels import paged_attention_integration as integration
 from engine.kernels.paged_attention_integration import (
     DECODE_LINEAR_MAX_ROWS,
     PagedAttentionContext,
     _ids_checked,
+    _max_rows,
     _stack_takes,
     _weights_readable,
 )
@@ -133,3 +135,41 @@ def test_weights_the_kernels_cannot_read_take_the_layers():
     m = layer()
     m.input_layernorm.weight = torch.zeros(65, **half)[1:]
     assert not _weights_readable(m)
+
+
+def _layer(hidden, mlp, heads, kv_heads, dim):
+    """A prepared layer of these sizes without storage."""
+    empty = lambda *shape: torch.empty(shape, dtype=torch.float16, device="meta")  # noqa: E731
+    qkv = (heads + 2 * kv_heads) * dim
+    return SimpleNamespace(
+        self_attn=SimpleNamespace(o_proj=SimpleNamespace(weight=empty(hidden, heads * dim))),
+        mlp=SimpleNamespace(down_proj=SimpleNamespace(weight=empty(hidden, mlp))),
+        _pa_packed=(empty(qkv // 16, hidden // 32, 4, 16, 8),
+                    empty(2 * mlp // 16, hidden // 32, 4, 16, 8)))
+
+
+# The sizes measured beside DECODE_LINEAR_ROWS: up to the last row count at which the stack was not
+# the slower path, or fewer.
+@pytest.mark.parametrize("sizes,rows", [
+    ((896, 4864, 14, 2, 64), 256), ((1536, 8960, 12, 2, 128), 128), ((2048, 5504, 16, 16, 128), 128),
+    ((2048, 11008, 16, 2, 128), 128), ((2560, 9728, 32, 8, 128), 128),
+    ((4096, 11008, 32, 32, 128), 64), ((3584, 18944, 28, 4, 128), 64),
+    ((5120, 27648, 40, 8, 128), 64), ((8192, 29568, 64, 8, 128), 32)])
+def test_rows_by_layer_size(sizes, rows):
+    assert _max_rows(_layer(*sizes)) == rows
+
+
+def test_more_rows_than_the_layers_size_allows_take_the_layers(model, monkeypatch):
+    monkeypatch.setattr(model, "_orig_stack_forward", lambda **kwargs: "layers", raising=False)
+    monkeypatch.setattr(integration, "_weights_readable", lambda layer: True)
+    monkeypatch.setattr(integration, "_max_rows", lambda layer: 16 if layer is model.layers[1] else 64)
+    monkeypatch.setattr(integration, "_plain_embedding_and_rope", lambda m: 1 / 0)  # the stack itself
+
+    def call(rows):
+        ids = torch.zeros(rows, 1, dtype=torch.long)
+        return integration.fused_decoder_stack_forward(model, input_ids=ids, position_ids=ids,
+                                                       use_cache=False)
+
+    assert call(17) == "layers"
+    with pytest.raises(ZeroDivisionError):
+        call(16)

@@ -666,11 +666,28 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 # ---- the decode step's projections over packed operands -------------------------
 
-# Rows up to which a decode step's projections take pa_decode_linear_f16: a layer's
-# four launches against the library GEMMs with their norm and SwiGLU launches,
-# measured in captured graphs on the 0.5B-class model: 128 rows 27 against 59 us,
-# 256 rows 39 against about 53; at 512 rows 67 against 62.
+# Rows up to which a decode step's projections take pa_decode_linear_f16, by the weights of
+# a layer: the kernel shares nothing between workgroups but the L2s, so the larger the layer,
+# the fewer rows until the library's products, staged through LDS, make up for their three norm
+# and SwiGLU launches. A whole decode step per layer against the layer path, captured graphs, us
+# (hidden / MLP, heads; millions of weights):
+#   896 / 4864, 14 / 2 x 64 (15M): 8 rows 28 against 57, 128 39 / 68, 256 55 / 75 (512 rows, four
+#     projections alone, 67 / 62)
+#   1024 / 2816, 16 / 16 x 64 (13M): 64 49 / 84, 256 100 / 126
+#   1536 / 8960, 12 / 2 x 128 (47M): 64 57 / 94, 192 119 / 123, 256 127 / 129
+#   2048 / 5504, 16 / 16 x 128 (51M): 64 86 / 121, 128 119 / 146, 192 182 / 179
+#   2048 / 11008, 16 / 2 x 128 (77M): 64 75 / 117, 128 104 / 121, 192 154 / 150
+#   2560 / 9728, 32 / 8 x 128 (101M): 64 108 / 139, 128 169 / 191, 192 207 / 191
+#   4096 / 11008, 32 / 32 x 128 (202M): 64 183 / 214, 80 249 / 233, 128 306 / 299
+#   3584 / 18944, 28 / 4 x 128 (233M): 64 164 / 237, 128 262 / 283, 192 335 / 324
+#   5120 / 27648, 40 / 8 x 128 (488M): 64 349 / 388, 96 394 / 425, 128 484 / 457
+#   8192 / 29568, 64 / 8 x 128 (878M): 1 341 / 436, 64 520 / 522, 80 651 / 598
+# with 64 tokens of context; with 3000, where the attention takes most of the time and is
+# not followed by fetched weights, the stack is 1.04 (2048 / 5504, 128 rows) to 1.96 times as
+# fast at the row counts below.
 DECODE_LINEAR_MAX_ROWS = 256
+DECODE_LINEAR_ROWS = ((32 << 20, DECODE_LINEAR_MAX_ROWS), (110 << 20, 128), (512 << 20, 64),
+                      (math.inf, 32))
 
 
 def _packable(weight: torch.Tensor) -> bool:
@@ -1001,6 +1018,13 @@ def _weights_readable(layer: nn.Module) -> bool:
                     for m in (layer.input_layernorm, layer.post_attention_layernorm)))
 
 
+def _max_rows(layer: nn.Module) -> int:
+    """Rows up to which a prepared layer's projections take the packed kernels."""
+    values = sum(w.numel() for w in (*layer._pa_packed, layer.self_attn.o_proj.weight,
+                                     layer.mlp.down_proj.weight))
+    return next(rows for most, rows in DECODE_LINEAR_ROWS if values <= most)
+
+
 def fused_decoder_stack_forward(
     self: nn.Module,
     input_ids: Optional[torch.Tensor] = None,
@@ -1018,12 +1042,13 @@ def fused_decoder_stack_forward(
     RoPE, K/V write and paged attention; o + residual; post-attention norm +
     gate/up + SwiGLU; down + residual. Calls that ask for more than a decode
     step's hidden states (masks, caches, hidden-state outputs, tuples), layers with
-    forward hooks, weights the kernels cannot read and more than
-    DECODE_LINEAR_MAX_ROWS rows take the layers one by one as before.
+    forward hooks, weights the kernels cannot read and more rows than
+    DECODE_LINEAR_ROWS gives the layers' size take the layers one by one as before.
     """
     if not _stack_takes(self, input_ids, attention_mask, position_ids, past_key_values,
                         inputs_embeds, use_cache, kwargs) or \
-            not all(_weights_readable(layer) for layer in self.layers):
+            not all(_weights_readable(layer) and input_ids.shape[0] <= _max_rows(layer)
+                    for layer in self.layers):
         return self._orig_stack_forward(input_ids=input_ids, attention_mask=attention_mask,
                                         position_ids=position_ids, past_key_values=past_key_values,
                                         inputs_embeds=inputs_embeds, use_cache=use_cache, **kwargs)
