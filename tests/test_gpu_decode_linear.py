@@ -222,6 +222,38 @@ def test_o_and_down_follow_their_parameters(cuda_device, use_graphs):
     assert (new - old).norm() >= 0.1 * want.norm()
 
 
+def test_packed_copies_only_where_memory_is_left(cuda_device, monkeypatch):
+    """All layers' packed copies within a quarter of the free memory, or none: the step then runs
+    layer by layer. A later runner packs them if it finds the room."""
+    from engine import workloads
+    from engine.kernels import paged_attention_integration as integration
+    from engine.memory.block_allocator import BlockTable
+
+    config = dict(vocab_size=512, hidden_size=128, intermediate_size=256, num_hidden_layers=2,
+                  num_attention_heads=4, num_key_value_heads=2, max_position_embeddings=4096,
+                  rope_theta=1e6, tie_word_embeddings=False)
+    copies = 2 * 2 * (256 * 128 + 512 * 128)  # two layers' q/k/v and gate/up, two bytes each
+    free = integration._free_bytes(cuda_device)
+    held = torch.empty(64 << 20, dtype=torch.uint8, device=cuda_device)
+    assert 0 <= free - integration._free_bytes(cuda_device) - held.numel() <= 16 << 20
+    with torch.inference_mode():
+        model = workloads.decode_model(cuda_device, 14, config)
+        logits = []
+        for room, packed in ((4 * copies - 1, False), (4 * copies, True)):
+            monkeypatch.setattr(integration, "_free_bytes", lambda device: room)
+            runner = integration.KernelPagedManualDecode(model, num_blocks=4,
+                                                         device=str(cuda_device))
+            assert all(hasattr(m, "_pa_fused") and hasattr(m, "_pa_packed") == packed
+                       for m in model.model.layers)
+            for c in runner.pool.k_cache + runner.pool.v_cache:
+                c.zero_()
+            seq = {"seq_id": 0, "block_table": BlockTable(0, 16, [3], 5), "last_token_id": 9}
+            runner.decode_step([seq])
+            logits.append(seq["last_logits"].float())
+    # Two layers of fp16 activations: some fourteen roundings of 2^-11.
+    assert (logits[0] - logits[1]).norm() <= 14 * 2.0 ** -11 * logits[0].norm()
+
+
 @pytest.mark.parametrize("use_graphs", [False, True])
 def test_ids_nobody_checked_go_through_the_embedding_module(cuda_device, monkeypatch, use_graphs):
     """decode_step refuses ids outside the table and embeds the others in the step's first launch; a

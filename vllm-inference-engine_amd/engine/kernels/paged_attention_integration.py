@@ -841,22 +841,42 @@ def _is_decoder_layer(m: nn.Module) -> bool:
             and hasattr(m, "input_layernorm") and hasattr(m, "post_attention_layernorm"))
 
 
+def _free_bytes(device: torch.device) -> int:
+    """Device memory a new tensor can come from: the driver's and torch's own unused blocks."""
+    return (torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device)
+            - torch.cuda.memory_allocated(device))
+
+
+def _packed_weights(layer: nn.Module) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """The merged weights of a prepared layer whose projections suit the packed kernels."""
+    attn, mlp = layer.self_attn, layer.mlp
+    qkv, _, gate_up = layer._pa_fused
+    weights = (qkv, attn.o_proj.weight, gate_up, mlp.down_proj.weight)
+    if all(w.is_cuda and _packable(w) for w in weights) and \
+            qkv.shape[1] % 32 == 0 and mlp.down_proj.weight.shape[0] % 32 == 0:
+        return qkv, gate_up
+    return None
+
+
 def prepare_fused_layers(model: nn.Module) -> int:
     """Concatenate each decoder layer's q/k/v and gate/up weights once, for the fused decode path.
 
     The merged copies live on the layer (`_pa_fused`); the model's own modules
     are left as they are. Where the sizes allow it, the merged weights are also
     kept in the packed layout of the decode-step kernels (`_pa_packed`: q/k/v,
-    gate/up; fused_decoder_stack_forward). Returns the number of layers prepared.
+    gate/up; fused_decoder_stack_forward), unless these further copies of all
+    layers would take more than a quarter of the memory that is still free: the
+    layers work without them. Returns the number of layers prepared.
     Inference only: the copies do not follow later changes of the weights; o and
     down are read from the model's own parameters by every path.
     """
     n = 0
     if not isinstance(model, nn.Module):
         return n
+    layers = [m for m in model.modules() if _is_decoder_layer(m)]
     with torch.no_grad():
-        for m in model.modules():
-            if not _is_decoder_layer(m) or hasattr(m, "_pa_fused"):
+        for m in layers:
+            if hasattr(m, "_pa_fused"):
                 continue
             attn, mlp = m.self_attn, m.mlp
             if getattr(mlp, "act_fn", None) is not None and \
@@ -871,11 +891,17 @@ def prepare_fused_layers(model: nn.Module) -> int:
                 qkv_b,
                 torch.cat([mlp.gate_proj.weight, mlp.up_proj.weight]).contiguous(),
             )
-            weights = (m._pa_fused[0], attn.o_proj.weight, m._pa_fused[2], mlp.down_proj.weight)
-            if all(w.is_cuda and _packable(w) for w in weights) and \
-                    weights[0].shape[1] % 32 == 0 and weights[3].shape[0] % 32 == 0:
-                m._pa_packed = (pack_weight(weights[0]), pack_weight(weights[2]))
             n += 1
+        todo: Dict[torch.device, list] = {}
+        for m in layers:
+            if hasattr(m, "_pa_fused") and not hasattr(m, "_pa_packed"):
+                merged = _packed_weights(m)
+                if merged is not None:
+                    todo.setdefault(merged[0].device, []).append((m, merged))
+        for device, group in todo.items():
+            if sum(2 * w.numel() for _, merged in group for w in merged) <= _free_bytes(device) // 4:
+                for m, merged in group:
+                    m._pa_packed = tuple(pack_weight(w) for w in merged)
     return n
 
 
