@@ -252,17 +252,21 @@ constexpr int kPairShortTiles = 64;
 constexpr int kSkMinRange = 16;
 // Batches of at most this many pairs (at head_dim 128 and 256: kSkFewPairsWide)
 // take the kernel for few pairs, whose merges split a pair's rounds of records
-// over the threads, and at most kSkFewRanges ranges per pair: each more is
-// another record to merge. Measured on MI355X (launches in a captured graph,
-// two pools in turn, 14 q / 2 kv heads of 64 unless stated), the general kernel
-// against it, us: 1 x 2048 tokens 14.1 and 12.9, 8192 18.3 and 14.5, 24001 28.2
-// and 16.6, 32768 30.9 and 15.0; 2 x 12000 21.4 and 16.5; 4 x up to 16384 19.8
-// and 15.4; 8 x up to 3001 13.2 and 12.0; 60 x up to 4096 (120 pairs) 22.8 and
-// 22.5; head_dim 32, 16384 tokens 21.4 and 13.9; head_dim 256 31.3 and 29.3; 4
-// kv heads of 128, 24000 tokens 22.9 and 20.4, but 32 pairs of 6000 27.2 and
-// 27.6, 64 of up to 8192 32.6 and 33.0. Ranges per pair, 24, 32, 48, 64, 96:
-// 24001 tokens 18.1, 17.1, 16.6, 17.1, 18.1; 32768 17.9, 16.0, 15.0, 15.3, 16.4;
-// shorter contexts within 0.5 (their ranges are kSkMinRange positions).
+// over the threads, and at most kSkFewRanges ranges per pair on average (the
+// total is capped: one long context among short ones is cut more finely): each
+// more is another record to merge. Measured on MI355X (launches in a captured
+// graph, two pools in turn, 14 q / 2 kv heads of 64 unless stated), the general
+// kernel against it, us: 1 x 2048 tokens 14.1 and 12.9, 8192 18.3 and 14.5, 24001
+// 28.2 and 16.6, 32768 30.9 and 15.0; 2 x 12000 21.4 and 16.5; 4 x up to 16384
+// 19.8 and 15.4; 8 x up to 3001 13.2 and 12.0; 60 x up to 4096 (120 pairs) 22.8
+// and 22.5; at the limit of 256 pairs (8 kv heads of 64) 32 x 4096 57.7 and 57.2,
+// 8192 111.6 and 110.3, up to 8192 56.1 and 55.8, one of 16384 with 31 of up to
+// 64 21.6 and 20.7 (the last with 59 others at 2 kv heads 17.9 and 13.9);
+// head_dim 32, 16384 tokens 21.4 and 13.9; head_dim 256 31.3 and 29.3; 4 kv heads
+// of 128, 24000 tokens 22.9 and 20.4, but 32 pairs of 6000 27.2 and 27.6, 64 of
+// up to 8192 32.6 and 33.0. Ranges per pair, 24, 32, 48, 64, 96: 24001 tokens
+// 18.1, 17.1, 16.6, 17.1, 18.1; 32768 17.9, 16.0, 15.0, 15.3, 16.4; shorter
+// contexts within 0.5 (their ranges are kSkMinRange positions).
 constexpr int kSkFewPairs = 256;
 constexpr int kSkFewPairsWide = 16;
 constexpr int kSkFewRanges = 48;
