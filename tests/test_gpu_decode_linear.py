@@ -34,8 +34,8 @@ def _within(got, want, terms, rel_terms):
     assert worst <= 1.0
 
 
-# Row counts at the edges of the 16-row tiles; sizes whose tile counts leave remainders for
-# every tile shape, K from one step (most wavefronts idle) through both wavefront counts.
+# Row counts at the edges of the 16-row tiles, K from one step (most wavefronts idle) through both
+# wavefront counts; tiles past the end of N or M: test_tiles_past_the_end.
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 100, 128, 256])
 @pytest.mark.parametrize("n,k", [(32, 32), (1152, 896), (80, 2336), (896, 4864)])
 def test_linear_with_bias_residual_and_sums(cuda_device, rows, n, k):
@@ -57,9 +57,8 @@ def test_linear_with_bias_residual_and_sums(cuda_device, rows, n, k):
     assert out.sums.shape == (n // 16, rows)
 
 
-# Row-major weights, loaded four K steps at a time: K of fewer steps than wavefronts, ranges that end
-# inside a block of four, both wavefront counts; column tiles (71 and 72 of them) and row tiles that
-# leave remainders for every tile shape; rows of a wider buffer.
+# Row-major weights, loaded two K steps at a time: K of fewer steps than wavefronts, ranges that end
+# inside a pair, both wavefront counts; rows of a wider buffer.
 @pytest.mark.parametrize("rows", [1, 17, 50, 100, 128, 241, 256])
 @pytest.mark.parametrize("n,k", [(32, 32), (1136, 96), (1152, 896), (1136, 2336), (896, 4864)])
 def test_row_major_weights(cuda_device, rows, n, k):
@@ -81,6 +80,87 @@ def test_row_major_weights(cuda_device, rows, n, k):
     _within(out.unpack(), want + res.double(), terms + res.double().abs(), (k + 1) * 2.0 ** -24)
     squares = out.unpack().double().square()
     assert torch.allclose(out.sums.double().sum(0), squares.sum(1), rtol=n * 2.0 ** -24, atol=0)
+
+
+def _tile(kind, rows, n, k, cus=256):
+    """The dispatch of launch_decode_linear: (wavefronts, column tiles, row tiles) of a workgroup."""
+    mt, nt, up = -(-rows // 16), n // 16, lambda a, b: -(-a // b)  # noqa: E731
+    if kind == "silu":
+        if mt == 1 or mt * up(nt, 2) <= cus:
+            return 4, 2, 1
+        if mt == 2 or up(mt, 2) * up(nt, 2) <= cus:
+            return 4, 2, 2
+        return (4, 3, 2) if mt == 3 or up(mt, 2) * up(nt, 3) <= cus else (4, 3, 4)
+    nw = 8 if k > 32 * 4 * 14 else 4
+    if mt * nt <= cus:
+        return nw, 1, 1
+    if kind == "row" and nw == 8:
+        if mt > 1 and up(mt, 2) * nt <= cus:
+            return nw, 1, 2
+        return (nw, 2, 1) if mt == 1 else (nw, 2, 2)
+    return (nw, 2, 1) if mt == 1 or mt * up(nt, 2) <= cus else (nw, 2, 2)
+
+
+# (kind, rows, n, k): every kernel of the dispatch, with columns and rows of tiles past the end of N
+# and M wherever its tile has more than one.
+_PAST_THE_END = [
+    *(("plain", rows, 1136, k) for rows in (3, 100, 200) for k in (96, 2336)),
+    *(("norm", rows, 1136, k) for rows in (3, 100, 200) for k in (96, 2304)),
+    *(("row", rows, 1136, k) for rows in (3, 100, 200) for k in (96, 2336)),
+    ("row", 70, 1136, 2336), ("row", 5, 4112, 2336),
+    ("silu", 100, 1136, 96), ("silu", 140, 1136, 96), ("silu", 200, 1184, 96),
+    ("silu", 200, 4864, 896),
+]
+
+
+def test_every_kernel_runs_past_the_end():
+    """_PAST_THE_END against the dispatch: each kernel once with a remainder in N and in M."""
+    tiles = {(1, 1), (2, 1), (2, 2)}
+    want = {(kind, nw, *t) for kind in ("plain", "norm", "row") for nw in (4, 8) for t in tiles}
+    want |= {("row", 8, 1, 2), ("silu", 4, 2, 1), ("silu", 4, 2, 2), ("silu", 4, 3, 2),
+             ("silu", 4, 3, 4)}
+    columns, rows_ = set(), set()
+    for kind, rows, n, k in _PAST_THE_END:
+        tile = _tile(kind, rows, n, k)
+        if tile[1] == 1 or n // 16 % tile[1]:
+            columns.add((kind, *tile))
+        if rows % 16 and (tile[2] == 1 or -(-rows // 16) % tile[2]):
+            rows_.add((kind, *tile))
+    assert columns == want and rows_ == want
+
+
+@pytest.mark.parametrize("kind,rows,n,k", _PAST_THE_END)
+def test_tiles_past_the_end(cuda_device, kind, rows, n, k):
+    """Row-major outputs: packed ones have whole pairs of column tiles."""
+    assert torch.cuda.get_device_properties(cuda_device).multi_processor_count == 256
+    x, w, g = _data(rows, 2 * n if kind == "silu" else n, k, cuda_device, rows + n + k)
+    gain = torch.randn(k, generator=g, device=cuda_device).half()
+    xd = x.double()
+    rel = k * 2.0 ** -24
+    if kind in ("norm", "silu"):
+        xd = xd * torch.rsqrt(xd.square().mean(1, keepdim=True) + EPS) * gain.double()
+        rel = 2.0 ** -11 + (k + 8) * 2.0 ** -24
+    want, terms = xd @ w.double().t(), xd.abs() @ w.double().abs().t()
+    packed = pack_rows(x)
+    norm = (gain, EPS) if kind in ("norm", "silu") else None
+    got = decode_linear(packed, w if kind == "row" else pack_weight(w), norm=norm,
+                        silu=kind == "silu", packed=False)
+    # Operands below fp16's normal range are rounded to a multiple of 2^-24 of the scaled row.
+    small = w.double().abs().sum(1)[None, :] * 2.0 ** -24 if norm else torch.zeros_like(want)
+    if kind != "silu":
+        _within(got, want, terms + small / rel, rel)
+        if kind != "norm":
+            assert torch.equal(got, decode_linear(x, w if kind == "row" else pack_weight(w),
+                                                  packed=False))
+        return
+    gate, up = want[:, :n], want[:, n:]
+    err = rel * terms + small
+    want = torch.nn.functional.silu(gate) * up
+    bound = 1.1 * err[:, :n] * (up.abs() + err[:, n:]) + gate.abs() * err[:, n:]
+    _within(got, want, bound + want.abs() * 2.0 ** -21, 1.0)
+    if n % 32 == 0:
+        out = decode_linear(packed, pack_weight(w), norm=norm, silu=True)
+        assert torch.equal(out.unpack(), got)
 
 
 @pytest.mark.parametrize("rows", [1, 16, 31, 48, 64, 100, 128, 256])
