@@ -1305,9 +1305,9 @@ struct PairSeg {
 //
 // A small batch's attention leaves most CUs and the memory idle for its 9 us,
 // and the projections after it are bound by their weight streams: read from L2
-// they take (8 rows, hidden 896) 4.3 instead of 6.6 us (gate/up), 4.4 instead of
-// 5.5 (down), 2.9 instead of 3.2 (o); at 128 rows 8.1 instead of 10.8, 5.9
-// instead of 7.0, 4.1 instead of 4.5. Whole decode steps: 8 streams 919 -> 820
+// they take (8 rows, hidden 896) 4.3 instead of 6.6 us (gate/up), 5.2 instead of
+// 6.2 (down, row-major), 3.1 instead of 3.5 (o); at 128 rows 8.1 instead of 10.8, 6.9
+// instead of 7.8, 3.9 instead of 4.3. Whole steps (o and down packed): 8 streams 919 -> 820
 // us, 128 streams (whose attention fills the CUs) 1363 -> 1324. The parts match
 // the consumers' workgroup order (xcd_order over column tiles); L2 contents
 // stay across launches.
