@@ -59,8 +59,9 @@ enum {
  * schedule plan that pa_decode_kv_write_batched_f16's write launch leaves for its
  * attention launch, 8,448 bytes more; 15: pa_pack_rows_f16, pa_decode_linear_f16;
  * 16: pa_decode_embed_f16; 17: pa_greedy_f16; 18:
- * pa_decode_rope_prefetch_f16; 19: weight_row_stride of pa_decode_linear_f16).
- * pa_abi_version returns the library's. */
+ * pa_decode_rope_prefetch_f16; 19: weight_row_stride of pa_decode_linear_f16, a
+ * rotary workspace that never holds queries in the counter region). pa_abi_version
+ * returns the library's. */
 #define PA_ABI_VERSION 19
 PA_API int pa_abi_version(void);
 

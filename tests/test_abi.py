@@ -45,6 +45,18 @@ def _device_cus():
     return 256
 
 
+def test_rotated_queries_stay_behind_the_counters():
+    """Also where the attention call itself needs no workspace (more than 1024 short sequences):
+    the counters must still be zero for the next call on the same workspace."""
+    lib = _native.load()
+    counters = 65536 * 4 + (2 * 1024 + 64) * 4
+    for seqs, blocks in ((1025, 1), (1065, 14), (4000, 8), (1025, 2048), (8, 64)):
+        for hq, hkv, d in ((4, 2, 32), (14, 2, 64), (28, 4, 128)):
+            own = lib.pa_decode_batched_workspace_bytes(seqs, hq, hkv, d, 16, blocks)
+            rope = lib.pa_decode_rope_batched_workspace_bytes(seqs, hq, hkv, d, 16, blocks)
+            assert rope >= max(own, counters) + seqs * hq * d * 2
+
+
 def test_workspace_sizes():
     lib = _native.load()
     cus = _device_cus()

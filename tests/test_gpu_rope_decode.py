@@ -112,3 +112,22 @@ def test_repeated_calls_are_bit_identical(cuda_device):
                                     c["lens"], c["scale"])
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+def test_many_short_sequences_leave_the_workspace_as_they_found_it(cuda_device):
+    """More than 1024 sequences in one split each: the attention call uses no workspace, the rotated
+    queries do, and stream-K calls after it count from zero."""
+    from engine.kernels import _native
+
+    rng = np.random.default_rng(4)
+    many = make_case(1030, 4, 2, 32, 16, lens_for(1030, rng, 1, 60, 16), 11, cuda_device)
+    few = make_case(8, 14, 2, 64, 16, lens_for(8, rng, 64, 2000, 16), 12, cuda_device)
+    call = lambda c: paged_attention_decode_batched(  # noqa: E731
+        c["q"], c["kc"], c["vc"], c["bt"], c["lens"], c["scale"])
+    before = call(few)
+    got, want, _, _, _ = run_both(many)
+    assert torch.equal(got, want)
+    key = (cuda_device.index, _native.stream_handle(cuda_device), _native.WS_DECODE)
+    counters = _native._workspaces[key][:65536 * 4]
+    assert torch.count_nonzero(counters).item() == 0
+    assert torch.equal(call(few), before)

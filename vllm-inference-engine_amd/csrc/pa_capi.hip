@@ -987,6 +987,13 @@ int pa_rope_kv_write_f16(const void* q, const int64_t q_strides[3], const void* 
   return finish_launch(launch_rope_kv_write(a, vec, (hipStream_t)stream));
 }
 
+// Where the rotated queries of the two-launch rotary form start: behind the decode workspace, and
+// behind its counter region also where the attention call uses none (fixed split, one split per
+// sequence): later calls on the same workspace rely on its zeros.
+static size_t rope_rows_offset(size_t decode_ws) {
+  return ((decode_ws > kSkCounterBytes ? decode_ws : kSkCounterBytes) + 255) & ~(size_t)255;
+}
+
 size_t pa_decode_rope_batched_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads,
                                               int head_dim, int block_size,
                                               int max_blocks_per_seq) {
@@ -997,7 +1004,7 @@ size_t pa_decode_rope_batched_workspace_bytes(int num_seqs, int num_q_heads, int
   // form (used when the one-launch kernel does not serve the shape).
   const size_t ws = pa_decode_batched_workspace_bytes(num_seqs, num_q_heads, num_kv_heads,
                                                       head_dim, block_size, max_blocks_per_seq);
-  return ((ws + 255) & ~(size_t)255) + (size_t)num_seqs * num_q_heads * head_dim * 2;
+  return rope_rows_offset(ws) + (size_t)num_seqs * num_q_heads * head_dim * 2;
 }
 
 static int rope_batched(const void* q, const int64_t q_strides[3], const void* key,
@@ -1085,7 +1092,7 @@ static int rope_batched(const void* q, const int64_t q_strides[3], const void* k
       out_strides[2] == 1 && out_strides[0] % 4 == 0 && out_strides[1] % 4 == 0;
   if (!one_launch) {
     // Two launches: rotation and K/V write, then attention on the rotated queries.
-    void* q_rot = (char*)workspace + ((dec_ws + 255) & ~(size_t)255);
+    void* q_rot = (char*)workspace + rope_rows_offset(dec_ws);
     const int64_t qr_strides[3] = {(int64_t)num_q_heads * head_dim, head_dim, 1};
     rc = pa_rope_kv_write_f16(q, q_strides, key, key_strides, value, value_strides, cos, cos_strides,
                               sin, sin_strides, q_rot, qr_strides, k_cache, k_strides, v_cache,
