@@ -151,9 +151,14 @@ __global__ __launch_bounds__(64 * NW) void decode_linear_kernel(LinearArgs a) {
     for (int i = 0; i < TN; ++i) {
       *reinterpret_cast<u32x4*>(&s_w[w_put + i * kTile]) = wf[j][i];
       *reinterpret_cast<u32x4*>(&s_w[w_put + i * kTile + 8 * 16]) = wf[j + 1][i];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
       wf[j][i] = *reinterpret_cast<const u32x4*>(&s_w[w_get + i * kTile]);
       wf[j + 1][i] = *reinterpret_cast<const u32x4*>(&s_w[w_get + i * kTile + 4 * kPiece]);
     }
+    wave_lds_fence();
   };
   auto load = [&](int j, int u) {
     const int nb = u < u1 ? 0x7fffffff : 0;
