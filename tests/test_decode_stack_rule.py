@@ -11,9 +11,9 @@ from engine.kernels.paged_attention_integration import (
     DECODE_LINEAR_MAX_ROWS,
     PagedAttentionContext,
     _ids_checked,
-    _max_rows,
+    _stack_layer,
+    _stack_sizes,
     _stack_takes,
-    _weights_readable,
 )
 
 
@@ -102,50 +102,56 @@ def test_only_ids_checked_against_the_table_skip_the_embedding_module():
         assert _ids_checked(ctx, emb) == taken
 
 
+def _packed_layer():
+    """A decoder layer with the sizes that the packed copies leave on it (no copies needed here)."""
+    from transformers import Qwen2Config
+    from transformers.models.qwen2.modeling_qwen2 import Qwen2DecoderLayer
+
+    layer = Qwen2DecoderLayer(Qwen2Config(hidden_size=64, intermediate_size=96,
+                                          num_attention_heads=2, num_key_value_heads=1,
+                                          head_dim=16), 0).half()
+    layer._pa_packed = (torch.zeros(1, dtype=torch.float16),) * 4
+    layer._pa_sizes = _stack_sizes(layer)
+    return layer
+
+
 def test_weights_the_kernels_cannot_read_take_the_layers():
     """The parameters that the stack reads in place: another type, shape, stride or alignment."""
     half = dict(dtype=torch.float16)
+    good = _stack_layer(_packed_layer(), 3)
+    assert good.o.shape == (64, 32) and (good.q_width, good.kv_width) == (32, 16)
 
-    def layer():
-        linear = lambda n, k: SimpleNamespace(weight=torch.zeros(n, k, **half), bias=None,  # noqa: E731
-                                              out_features=n)
-        norm = lambda: SimpleNamespace(weight=torch.zeros(64, **half))  # noqa: E731
-        return SimpleNamespace(
-            self_attn=SimpleNamespace(o_proj=linear(64, 32), q_proj=linear(32, 64)),
-            mlp=SimpleNamespace(down_proj=linear(64, 96)), input_layernorm=norm(),
-            post_attention_layernorm=norm(),
-            _pa_packed=(torch.zeros(4, 2, 4, 16, 8, **half), torch.zeros(12, 2, 4, 16, 8, **half)))
+    def replaced(module, weight, name="weight"):
+        layer = _packed_layer()
+        owner = layer.get_submodule(module)
+        setattr(owner, name, torch.nn.Parameter(weight, requires_grad=False))
+        return _stack_layer(layer, 3)
 
-    assert _weights_readable(layer())
+    o, down, norm = "self_attn.o_proj", "mlp.down_proj", "input_layernorm"
     wide, odd = torch.zeros(64, 40, **half), torch.zeros(64 * 32 + 4, **half)
-    m = layer()
-    m.self_attn.o_proj.weight = wide[:, :32]
-    assert _weights_readable(m)
-    for name, weight in (("o_proj", torch.zeros(64, 32)), ("o_proj", torch.zeros(64, 64, **half)),
-                         ("o_proj", torch.zeros(32, 64, **half).t()),
-                         ("o_proj", torch.zeros(64, 36, **half)[:, :32]),
-                         ("o_proj", odd[4:].view(64, 32)),
-                         ("down_proj", torch.zeros(64, 64, **half))):
-        m = layer()
-        getattr(m.self_attn if name == "o_proj" else m.mlp, name).weight = weight
-        assert not _weights_readable(m)
-    m = layer()
-    m.self_attn.o_proj.bias = torch.zeros(64)
-    assert not _weights_readable(m)
-    m = layer()
-    m.input_layernorm.weight = torch.zeros(65, **half)[1:]
-    assert not _weights_readable(m)
+    assert replaced(o, wide[:, :32]).o.stride() == (40, 1)
+    assert replaced(o, torch.zeros(64, **half), "bias").o_bias is not None
+    for module, weight in ((o, torch.zeros(64, 32)), (o, torch.zeros(64, 64, **half)),
+                           (o, torch.zeros(32, 64, **half).t()),
+                           (o, torch.zeros(64, 36, **half)[:, :32]), (o, odd[4:].view(64, 32)),
+                           (down, torch.zeros(64, 64, **half)), (norm, torch.zeros(64)),
+                           (norm, torch.zeros(65, **half)[1:]), (norm, torch.zeros(128, **half)[::2])):
+        assert replaced(module, weight) is None
+    assert replaced(o, torch.zeros(64), "bias") is None
+    layer = _packed_layer()
+    torch.nn.utils.parametrize.register_parametrization(layer.mlp.down_proj, "weight",
+                                                        torch.nn.Identity())
+    assert _stack_layer(layer, 3) is None
 
 
 def _layer(hidden, mlp, heads, kv_heads, dim):
-    """A prepared layer of these sizes without storage."""
-    empty = lambda *shape: torch.empty(shape, dtype=torch.float16, device="meta")  # noqa: E731
-    qkv = (heads + 2 * kv_heads) * dim
+    """A layer of these sizes without storage."""
+    weight = lambda n, k: SimpleNamespace(  # noqa: E731
+        weight=torch.empty(n, k, dtype=torch.float16, device="meta"))
     return SimpleNamespace(
-        self_attn=SimpleNamespace(o_proj=SimpleNamespace(weight=empty(hidden, heads * dim))),
-        mlp=SimpleNamespace(down_proj=SimpleNamespace(weight=empty(hidden, mlp))),
-        _pa_packed=(empty(qkv // 16, hidden // 32, 4, 16, 8),
-                    empty(2 * mlp // 16, hidden // 32, 4, 16, 8)))
+        self_attn=SimpleNamespace(q_proj=weight(heads * dim, hidden),
+                                  k_proj=weight(kv_heads * dim, hidden)),
+        mlp=SimpleNamespace(down_proj=weight(hidden, mlp)))
 
 
 # The sizes measured beside DECODE_LINEAR_ROWS: up to the last row count at which the stack was not
@@ -156,18 +162,25 @@ def _layer(hidden, mlp, heads, kv_heads, dim):
     ((4096, 11008, 32, 32, 128), 64), ((3584, 18944, 28, 4, 128), 64),
     ((5120, 27648, 40, 8, 128), 64), ((8192, 29568, 64, 8, 128), 32)])
 def test_rows_by_layer_size(sizes, rows):
-    assert _max_rows(_layer(*sizes)) == rows
+    assert _stack_sizes(_layer(*sizes)).rows == rows
 
 
-def test_more_rows_than_the_layers_size_allows_take_the_layers(model, monkeypatch):
-    monkeypatch.setattr(model, "_orig_stack_forward", lambda **kwargs: "layers", raising=False)
-    monkeypatch.setattr(integration, "_weights_readable", lambda layer: True)
-    monkeypatch.setattr(integration, "_max_rows", lambda layer: 16 if layer is model.layers[1] else 64)
+def test_more_rows_than_the_layers_size_allows_take_the_layers(monkeypatch):
+    from transformers import Qwen2Config
+    from transformers.models.qwen2.modeling_qwen2 import Qwen2Model
+
+    m = Qwen2Model(Qwen2Config(vocab_size=32, hidden_size=64, intermediate_size=96,
+                               num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=1))
+    m._paged_stack_context = SimpleNamespace(is_decode=True, is_batched=True)
+    m._orig_stack_forward = lambda **kwargs: "layers"
+    for i in range(2):
+        m.layers[i] = _packed_layer()
+    m.layers[1]._pa_sizes = m.layers[1]._pa_sizes._replace(rows=16)
     monkeypatch.setattr(integration, "_plain_embedding_and_rope", lambda m: 1 / 0)  # the stack itself
 
     def call(rows):
         ids = torch.zeros(rows, 1, dtype=torch.long)
-        return integration.fused_decoder_stack_forward(model, input_ids=ids, position_ids=ids,
+        return integration.fused_decoder_stack_forward(m, input_ids=ids, position_ids=ids,
                                                        use_cache=False)
 
     assert call(17) == "layers"

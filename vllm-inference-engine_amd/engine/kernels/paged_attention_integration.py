@@ -30,7 +30,7 @@ import logging
 import math
 from collections import OrderedDict
 from contextlib import contextmanager
-from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple, Union
+from typing import Any, Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
@@ -785,8 +785,8 @@ def decode_linear(
     if asked) or, with packed=False, a row-major [rows, n] tensor.
     """
     if weight.dim() == 2:
-        (n, k), w_stride = weight.shape, weight.stride(0)
-        assert norm is None and not silu and _packable(weight) and weight.stride(1) == 1
+        (n, k), (w_stride, unit) = weight.shape, weight.stride()
+        assert unit == 1 and n % 16 == 0 and k % 32 == 0 and norm is None and not silu
     else:
         k, w_stride = weight.shape[1] * 32, 0
         n = weight.shape[0] * 16 // (2 if silu else 1)
@@ -901,7 +901,9 @@ def prepare_fused_layers(model: nn.Module) -> int:
         for device, group in todo.items():
             if sum(2 * w.numel() for _, merged in group for w in merged) <= _free_bytes(device) // 4:
                 for m, merged in group:
-                    m._pa_packed = tuple(pack_weight(w) for w in merged)
+                    qkv, gate_up = (pack_weight(w) for w in merged)
+                    m._pa_packed = (qkv, gate_up, *gate_up.chunk(2))  # and the halves to prefetch
+                    m._pa_sizes = _stack_sizes(m)
     return n
 
 
@@ -1023,32 +1025,72 @@ def _plain_embedding_and_rope(self: nn.Module) -> bool:
             and rope.inv_freq.is_contiguous())
 
 
-def _readable(t: torch.Tensor, shape: Tuple[int, ...], device: torch.device, align: int) -> bool:
-    """Whether the projection kernels read t where it is: fp16 of that shape, aligned rows."""
-    return (t.device == device and t.dtype == torch.float16 and t.shape == shape
-            and t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1])
-            and t.data_ptr() % align == 0)
+class _StackSizes(NamedTuple):
+    """Sizes of a packed layer, and the rows up to which its projections take the packed kernels."""
+
+    rows: int
+    hidden: int
+    inter: int
+    q_width: int
+    kv_width: int
 
 
-def _weights_readable(layer: nn.Module) -> bool:
-    """Whether a prepared layer's own parameters, as they now are, suit the fused stack."""
+def _stack_sizes(layer: nn.Module) -> _StackSizes:
     attn, mlp = layer.self_attn, layer.mlp
-    qkv, gate_up = layer._pa_packed
-    dev, hidden, inter = qkv.device, qkv.shape[1] * 32, gate_up.shape[0] * 8
-    width = attn.q_proj.out_features
-    bias = attn.o_proj.bias
-    return (_readable(attn.o_proj.weight, (hidden, width), dev, 16)
-            and _readable(mlp.down_proj.weight, (hidden, inter), dev, 16)
-            and (bias is None or _readable(bias, (hidden,), dev, 8))
-            and all(_readable(m.weight, (hidden,), dev, 16)
-                    for m in (layer.input_layernorm, layer.post_attention_layernorm)))
+    hidden, inter = mlp.down_proj.weight.shape
+    q_width, kv_width = attn.q_proj.weight.shape[0], attn.k_proj.weight.shape[0]
+    values = hidden * (2 * q_width + 2 * kv_width + 3 * inter)
+    rows = next(rows for most, rows in DECODE_LINEAR_ROWS if values <= most)
+    return _StackSizes(rows, hidden, inter, q_width, kv_width)
 
 
-def _max_rows(layer: nn.Module) -> int:
-    """Rows up to which a prepared layer's projections take the packed kernels."""
-    values = sum(w.numel() for w in (*layer._pa_packed, layer.self_attn.o_proj.weight,
-                                     layer.mlp.down_proj.weight))
-    return next(rows for most, rows in DECODE_LINEAR_ROWS if values <= most)
+def _readable(t: Any, shape: Tuple[int, ...], device: torch.device, align: int) -> bool:
+    """Whether the projection kernels read t where it is: fp16 of that shape, aligned rows."""
+    return (t is not None and t.dtype is torch.float16 and t.shape == shape and t.device == device
+            and t.data_ptr() % align == 0
+            and (t.is_contiguous() or (len(shape) == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0)))
+
+
+class _StackLayer(NamedTuple):
+    """What the fused stack reads of a layer: tensors, and the attention module."""
+
+    attn: nn.Module
+    qkv: torch.Tensor
+    gate_up: torch.Tensor
+    o: torch.Tensor
+    o_bias: Optional[torch.Tensor]
+    down: torch.Tensor
+    norm1: Tuple[torch.Tensor, float]
+    norm2: Tuple[torch.Tensor, float]
+    q_width: int
+    kv_width: int
+    fetch: List[torch.Tensor]  # what the launches after the attention read
+
+
+def _stack_layer(layer: nn.Module, rows: int) -> Optional[_StackLayer]:
+    """The packed layer as its parameters now are, or None where the stack does not serve it.
+
+    Read from the modules' own dictionaries: a step without a graph asks every
+    layer (a parameter that is computed, by a parametrisation, is not there).
+    """
+    sizes, (qkv, gate_up, gate, up) = layer._pa_sizes, layer._pa_packed
+    if rows > sizes.rows:
+        return None
+    mods = layer._modules
+    attn, norm1, norm2 = mods["self_attn"], mods["input_layernorm"], mods["post_attention_layernorm"]
+    o = attn._modules["o_proj"]._parameters
+    o_w, o_b = o.get("weight"), o.get("bias")
+    down = mods["mlp"]._modules["down_proj"]._parameters.get("weight")
+    w1, w2 = norm1._parameters.get("weight"), norm2._parameters.get("weight")
+    dev, vector = qkv.device, (sizes.hidden,)
+    if not (_readable(o_w, (sizes.hidden, sizes.q_width), dev, 16)
+            and _readable(down, (sizes.hidden, sizes.inter), dev, 16)
+            and _readable(w1, vector, dev, 16) and _readable(w2, vector, dev, 16)
+            and (o_b is None or _readable(o_b, vector, dev, 8))):
+        return None
+    fetch = [w for w in (o_w, gate, up, down) if w.is_contiguous()]
+    return _StackLayer(attn, qkv, gate_up, o_w, o_b, down, (w1, norm1.variance_epsilon),
+                       (w2, norm2.variance_epsilon), sizes.q_width, sizes.kv_width, fetch)
 
 
 def fused_decoder_stack_forward(
@@ -1071,10 +1113,12 @@ def fused_decoder_stack_forward(
     forward hooks, weights the kernels cannot read and more rows than
     DECODE_LINEAR_ROWS gives the layers' size take the layers one by one as before.
     """
-    if not _stack_takes(self, input_ids, attention_mask, position_ids, past_key_values,
-                        inputs_embeds, use_cache, kwargs) or \
-            not all(_weights_readable(layer) and input_ids.shape[0] <= _max_rows(layer)
-                    for layer in self.layers):
+    layers = None
+    if _stack_takes(self, input_ids, attention_mask, position_ids, past_key_values, inputs_embeds,
+                    use_cache, kwargs):
+        layers = [_stack_layer(layer, input_ids.shape[0])
+                  for layer in self.layers[:self.config.num_hidden_layers]]
+    if not layers or None in layers:
         return self._orig_stack_forward(input_ids=input_ids, attention_mask=attention_mask,
                                         position_ids=position_ids, past_key_values=past_key_values,
                                         inputs_embeds=inputs_embeds, use_cache=use_cache, **kwargs)
@@ -1082,7 +1126,6 @@ def fused_decoder_stack_forward(
 
     ctx = self._paged_stack_context
     b = input_ids.shape[0]
-    layers = self.layers[:self.config.num_hidden_layers]
     if position_ids.shape == (b, 1) and position_ids.dtype == input_ids.dtype == torch.int64 and \
             _plain_embedding_and_rope(self):
         rows, cos, sin = decode_embed(input_ids.reshape(b).contiguous(),
@@ -1094,25 +1137,21 @@ def fused_decoder_stack_forward(
         cos, sin = self.rotary_emb(x, position_ids)
         rows = pack_rows(x.view(b, -1))
     for i, layer in enumerate(layers):
-        attn, mlp = layer.self_attn, layer.mlp
-        qkv_w, gu_w = layer._pa_packed
-        o_w, down_w = attn.o_proj.weight, mlp.down_proj.weight
+        attn = layer.attn
         hd = attn.head_dim
-        nq = attn.q_proj.out_features // hd
-        nkv = attn.k_proj.out_features // hd
-        norm1, norm2 = layer.input_layernorm, layer.post_attention_layernorm
-        qkv = decode_linear(rows, qkv_w, norm=(norm1.weight, norm1.variance_epsilon),
-                            bias=layer._pa_fused[1], packed=False)
+        nq, nkv = layer.q_width // hd, layer.kv_width // hd
+        qkv = decode_linear(rows, layer.qkv, norm=layer.norm1, bias=self.layers[i]._pa_fused[1],
+                            packed=False)
         scale = attn.scaling if hasattr(attn, "scaling") else 1.0 / math.sqrt(hd)
         o = paged_rope_decode_attention(
             qkv[:, :nq * hd].view(b, nq, hd), qkv[:, nq * hd:(nq + nkv) * hd].view(b, nkv, hd),
             qkv[:, (nq + nkv) * hd:].view(b, nkv, hd), cos, sin, ctx.pool.k_cache[attn.layer_idx],
             ctx.pool.v_cache[attn.layer_idx], ctx.padded_block_tables, ctx.seq_lens_tensor, scale,
-            prefetch=[w for w in (o_w, *gu_w.chunk(2), down_w) if w.is_contiguous()])
-        h = decode_linear(o.view(b, nq * hd), o_w, bias=attn.o_proj.bias, residual=rows, sums=True)
-        act = decode_linear(h, gu_w, norm=(norm2.weight, norm2.variance_epsilon), silu=True)
+            prefetch=layer.fetch)
+        h = decode_linear(o.view(b, nq * hd), layer.o, bias=layer.o_bias, residual=rows, sums=True)
+        act = decode_linear(h, layer.gate_up, norm=layer.norm2, silu=True)
         last = i + 1 == len(layers)
-        rows = decode_linear(act, down_w, residual=h, packed=not last, sums=not last)
+        rows = decode_linear(act, layer.down, residual=h, packed=not last, sums=not last)
     return BaseModelOutputWithPast(last_hidden_state=self.norm(rows.view(b, 1, -1)))
 
 
@@ -1681,6 +1720,7 @@ class KernelPagedManualDecode:
                 block_table.physical_block_ids.append(alloc.allocate())
             block_table.num_tokens += 1
             ctx = PagedAttentionContext(self.pool, [block_table], [seq_len], self.block_size, True)
+            ctx.checked_vocab = history[-1].shape[-1]  # next_token is a position of these logits
             pos = torch.tensor([[seq_len - 1]], dtype=torch.long, device=self.device)
             with patch_paged_attention(self.model, ctx, fuse_layers=self.fuse_layers):
                 step = self.model(input_ids=next_token, position_ids=pos, use_cache=False)
